@@ -663,20 +663,171 @@ __global__ __launch_bounds__(BLOCK) void rank_segs(const kun_cs::Seg *segs) {
     rank_row_k<T, BLOCK, ITEMS, KIND>(in, out, g.n, 1, 0);
 }
 
-// ROWS rows per workgroup; the sum of each row is one sequential chain (lane
-// r of the first wave owns row r), fed from LDS tiles that the whole
-// workgroup loads one tile ahead and stores already masked: |x|, or +0 for a
-// NaN cell -- adding +0 to a sum of non-negative terms leaves it
-// bit-identical, so the chain is one dependent add per stock. LIN / LOUT are
-// the layouts (-1: read from the view at run time).
+// ---- Scale: row sums in stock order, a tile at a time ---------------------
 //
-// Many rows (batch runs): the sums go to scratch (4 rows per workgroup, the
-// chain being the bound) and a second kernel divides every cell on all CUs;
-// one row (stream ticks, pool segments): one workgroup sums and divides.
+// The reference adds |x| cell by cell, so the rounding of every add is part
+// of the result and the plain form is one dependent add per stock: 8.9 clocks
+// each on one wavefront, whatever else the GPU does. The sum of non-negative
+// terms has more structure. While the running sum s stays inside one binade
+// it is a multiple of one unit u, and adding x moves it by a whole number of
+// units that depends on s only through whether s / u is odd (round to nearest
+// even breaks a tie by that bit, and nothing else of s enters the rounding).
+// A run of consecutive cells is therefore a function of that one bit, found
+// by adding the run to the binade's first value and to the one after it, and
+// such functions compose. So:
+//  * a wavefront takes a tile of 64 x CHAIN_K cells, each lane CHAIN_K
+//    consecutive ones, and every lane adds its cells to both starting values;
+//  * a scan over the lanes composes the runs (a plain integer prefix sum
+//    unless some lane met a tie);
+//  * where the sum leaves the binade, the lanes before are taken, that lane's
+//    cells are added one by one, and the rest of the tile starts over in the
+//    new binade. The sum never falls, so a row leaves at most as many
+//    binades as the type has, and about 13 for 8192 cells of like size.
+// The result is the sequential sum bit for bit, infinities and subnormals
+// included (a subnormal sum's unit is the smallest subnormal).
+//
+// 1024 rows of 8192 floats: 16.3 us a launch (2.1 TB/s), bound by the tiles'
+// adds and scans on the one wavefront a SIMD has; the chain on one lane per
+// row took 49.5 us. 750 rows of 5003 doubles: 15.3 us against 34.6; one row
+// per session of a pool, about 2200 stocks, summed and divided: 10.3 us
+// against 24.5.
+constexpr int CHAIN_K = 16;
+constexpr int CHAIN_TILE = 64 * CHAIN_K;
+
+__device__ __forceinline__ uint32_t lane_value(uint32_t v, int l) {
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, l);
+}
+__device__ __forceinline__ uint64_t lane_value(uint64_t v, int l) {
+    return (uint64_t)lane_value((uint32_t)(v >> 32), l) << 32 | lane_value((uint32_t)v, l);
+}
+
+// the value CTRL brings from a lane before this one, 0 where there is none
+template <int CTRL, int ROWS> __device__ __forceinline__ uint32_t dpp_before(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
+}
+template <int CTRL, int ROWS> __device__ __forceinline__ uint64_t dpp_before(uint64_t v) {
+    return (uint64_t)dpp_before<CTRL, ROWS>((uint32_t)(v >> 32)) << 32 | dpp_before<CTRL, ROWS>((uint32_t)v);
+}
+
+// inclusive scan over the lanes of the runs' moves from an even (i0) and an
+// odd (i1) sum, in units
+template <int CTRL, int ROWS, typename U> __device__ __forceinline__ void compose_step(U &i0, U &i1) {
+    const U l0 = dpp_before<CTRL, ROWS>(i0), l1 = dpp_before<CTRL, ROWS>(i1);
+    const U r0 = l0 + ((l0 & 1) ? i1 : i0), r1 = l1 + ((l1 & 1) ? i0 : i1);
+    i0 = r0;
+    i1 = r1;
+}
+template <typename U> __device__ __forceinline__ void scan_runs(U &i0, U &i1) {
+    compose_step<0x111, 0xf>(i0, i1); // row_shr:1, 2, 4, 8, then row_bcast:15, 31
+    compose_step<0x112, 0xf>(i0, i1);
+    compose_step<0x114, 0xf>(i0, i1);
+    compose_step<0x118, 0xf>(i0, i1);
+    compose_step<0x142, 0xa>(i0, i1);
+    compose_step<0x143, 0xc>(i0, i1);
+}
+template <typename U> __device__ __forceinline__ U scan_units(U v) {
+    v += dpp_before<0x111, 0xf>(v);
+    v += dpp_before<0x112, 0xf>(v);
+    v += dpp_before<0x114, 0xf>(v);
+    v += dpp_before<0x118, 0xf>(v);
+    v += dpp_before<0x142, 0xa>(v);
+    v += dpp_before<0x143, 0xc>(v);
+    return v;
+}
+
+// s plus the 64 x CHAIN_K cells of a tile, added in order (lane l holds cells
+// l * CHAIN_K .. in v); v >= +0, not NaN; s is the same on every lane
+template <typename T> __device__ __forceinline__ T add_in_order(T s, const T (&v)[CHAIN_K]) {
+    using U = typename kun::Bits<T>::U;
+    constexpr U LIM = U(1) << kun::Bits<T>::MANT; // units in a binade
+    const int lane = threadIdx.x & 63;
+    for (int first = 0;;) {
+        const U sb = kun::to_bits(s);
+        if ((sb >> kun::Bits<T>::MANT) == (U(1) << kun::Bits<T>::EXPB) - 1) return s; // infinite: stays
+        const U b0 = sb & ~(LIM - 1);
+        T s0 = kun::from_bits<T>(b0), s1 = kun::from_bits<T>(b0 | 1);
+#pragma unroll
+        for (int k = 0; k < CHAIN_K; k++) {
+            s0 = s0 + v[k];
+            s1 = s1 + v[k];
+        }
+        // consecutive bit patterns are one unit apart; a run that leaves
+        // the binade counts as LIM, which no sum takes
+        U i0 = kun::to_bits(s0) - b0, i1 = kun::to_bits(s1) - (b0 | 1);
+        i0 = i0 < LIM ? i0 : LIM;
+        i1 = i1 < LIM ? i1 : LIM;
+        if (lane < first) i0 = i1 = 0;
+        U move;
+        if (__ballot(i0 != i1)) {
+            scan_runs(i0, i1);
+            move = (sb & 1) ? i1 : i0;
+        } else {
+            move = scan_units(i0);
+        }
+        const uint64_t leaves = __ballot((sb & (LIM - 1)) + move >= LIM);
+        if (!leaves) return kun::from_bits<T>(sb + lane_value(move, 63));
+        const int l = __builtin_ctzll(leaves);
+        T t = kun::from_bits<T>(l ? sb + lane_value(move, l - 1) : sb);
+#pragma unroll
+        for (int k = 0; k < CHAIN_K; k++) t = t + v[k];
+        s = kun::from_bits<T>(lane_value(kun::to_bits(t), l));
+        first = l + 1;
+        if (first == 64) return s;
+    }
+}
+
+// |x|, or +0 for a missing cell: adding +0 leaves the sum as it is
+template <typename T> __device__ __forceinline__ T scale_term(T x) { return x == x ? kun::vabs(x) : T(0); }
+
+// Sum of row `row` of the view, by one wavefront. Tiles are loaded two ahead
+// (coalesced) and turned lane by lane through LDS; the four cells of padding
+// per lane keep the reads of 16 bytes off each other's banks.
+template <typename T> struct ChainTile {
+    static constexpr int STRIDE = CHAIN_K + 16 / (int)sizeof(T);
+    alignas(16) T cell[64 * STRIDE];
+};
+template <typename T, int LIN>
+__device__ __forceinline__ T row_sum(ChainTile<T> &tile, const kun_cs::View &in, long row, long S, int blk) {
+    const int lane = threadIdx.x & 63;
+    const T *src = (const T *)in.ptr;
+    auto load = [&](T (&x)[CHAIN_K], long c0) {
+#pragma unroll
+        for (int j = 0; j < CHAIN_K; j++) {
+            const long s = c0 + j * 64 + lane;
+            x[j] = s < S ? src[lay_at<LIN>(in, row, s, S, blk)] : T(0);
+        }
+    };
+    T sum = T(0);
+    auto add = [&](const T (&x)[CHAIN_K]) {
+#pragma unroll
+        for (int j = 0; j < CHAIN_K; j++) {
+            const int e = j * 64 + lane;
+            tile.cell[e / CHAIN_K * ChainTile<T>::STRIDE + e % CHAIN_K] = scale_term(x[j]);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        T v[CHAIN_K];
+#pragma unroll
+        for (int k = 0; k < CHAIN_K; k++) v[k] = tile.cell[lane * ChainTile<T>::STRIDE + k];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        sum = add_in_order(sum, v);
+    };
+    T x[CHAIN_K], y[CHAIN_K];
+    load(x, 0);
+    load(y, CHAIN_TILE);
+    for (long c0 = 0; c0 < S; c0 += 2 * CHAIN_TILE) {
+        add(x);
+        load(x, c0 + 2 * CHAIN_TILE);
+        if (c0 + CHAIN_TILE < S) add(y);
+        load(y, c0 + 3 * CHAIN_TILE);
+    }
+    return sum;
+}
+
+// Many rows (batch runs): one wavefront per row leaves the sums in scratch
+// and a second kernel divides every cell on all CUs; one row (stream ticks,
+// pool segments): a workgroup whose first wavefront sums and which then
+// divides. LIN / LOUT are the layouts (-1: read from the view at run time).
 constexpr int SCALE_BLOCK = 256;
-constexpr int SCALE_ROWS = 8;
-constexpr int SCALE_SUM_ROWS = 4;
-constexpr int SCALE_TILE = 1024;
 
 // Scratch of the split form: the rows' sums, then (float rows) RN(1/sum) in
 // double at the next multiple of 8 bytes
@@ -694,85 +845,40 @@ __device__ __forceinline__ double scale_q(double x, double tot, double) {
     return (x == 0.0 && tot == 0.0) ? kun::qnan<double>() : x / tot;
 }
 
-// sums != null: store the row sums there (and their reciprocals, float)
-// and stop
-template <typename T, int LIN, int LOUT, int ROWS>
-__device__ __forceinline__ void scale_block(const kun_cs::View &in, const kun_cs::View &out, long S, long rows,
-                                            int blk, const long r0, T *sums) {
-    constexpr int PER = ROWS * SCALE_TILE / SCALE_BLOCK;
-    __shared__ T tile[ROWS * (SCALE_TILE + 1)];
-    __shared__ T total[ROWS];
-    const int nr = (int)((rows - r0) < ROWS ? (rows - r0) : ROWS);
+template <typename T, int LIN>
+__global__ __launch_bounds__(64) void scale_sums(kun_cs::View in, long S, long rows, int blk, T *sums) {
+    __shared__ ChainTile<T> tile;
+    const long r = blockIdx.x;
+    const T sum = row_sum<T, LIN>(tile, in, r + in.row0, S, blk);
+    if (threadIdx.x == 0) {
+        sums[r] = sum;
+        if (sizeof(T) == 4) scale_rcs(sums, rows)[r] = 1.0 / (double)sum;
+    }
+}
+
+// one row per workgroup, summed and divided
+template <typename T, int LIN, int LOUT>
+__device__ __forceinline__ void scale_row(const kun_cs::View &in, const kun_cs::View &out, long S, int blk, long r) {
+    __shared__ ChainTile<T> tile;
+    __shared__ T total;
+    if (threadIdx.x < 64) {
+        const T sum = row_sum<T, LIN>(tile, in, r + in.row0, S, blk);
+        if (threadIdx.x == 0) total = sum;
+    }
+    __syncthreads();
     const T *src = (const T *)in.ptr;
     T *dst = (T *)out.ptr;
-    T reg[PER];
-    auto load = [&](long c0) {
-#pragma unroll
-        for (int q = 0; q < PER; q++) {
-            const int e = threadIdx.x + q * SCALE_BLOCK;
-            const int r = e / SCALE_TILE, c = e % SCALE_TILE;
-            const long s = c0 + c;
-            reg[q] = (r < nr && s < S) ? src[lay_at<LIN>(in, r0 + r + in.row0, s, S, blk)] : T(0);
-        }
-    };
-    load(0);
-    T sum = T(0);
-    for (long c0 = 0; c0 < S; c0 += SCALE_TILE) {
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < PER; q++) {
-            const int e = threadIdx.x + q * SCALE_BLOCK;
-            const T x = reg[q];
-            tile[(e / SCALE_TILE) * (SCALE_TILE + 1) + e % SCALE_TILE] = (x == x) ? kun::vabs(x) : T(0);
-        }
-        __syncthreads();
-        if (c0 + SCALE_TILE < S) load(c0 + SCALE_TILE);
-        if ((int)threadIdx.x < nr) {
-            const int n = (int)((S - c0) < SCALE_TILE ? (S - c0) : SCALE_TILE);
-            const T *row = tile + threadIdx.x * (SCALE_TILE + 1);
-            // in stock order, as the reference's scalar loop; each group's
-            // LDS reads are issued before its adds, so their latency
-            // overlaps the chain
-            int k = 0;
-            for (; k + 16 <= n; k += 16) {
-                T g[16];
-#pragma unroll
-                for (int u = 0; u < 16; u++) g[u] = row[k + u];
-#pragma unroll
-                for (int u = 0; u < 16; u++) sum = sum + g[u];
-            }
-            for (; k < n; k++) sum = sum + row[k];
-        }
-    }
-    if (sums) {
-        if ((int)threadIdx.x < nr) {
-            sums[r0 + threadIdx.x] = sum;
-            if (sizeof(T) == 4) scale_rcs(sums, rows)[r0 + threadIdx.x] = 1.0 / (double)sum;
-        }
-        return;
-    }
-    if ((int)threadIdx.x < nr) total[threadIdx.x] = sum;
-    __syncthreads();
-    for (int r = 0; r < nr; r++) {
-        const T tot = total[r];
-        const double rc = sizeof(T) == 4 ? 1.0 / (double)tot : 0.0;
-        const long rr = r0 + r;
-        for (long s = threadIdx.x; s < S; s += SCALE_BLOCK) {
-            const T x = src[lay_at<LIN>(in, rr + in.row0, s, S, blk)];
-            dst[lay_at<LOUT>(out, rr + out.row0, s, S, blk)] = scale_q(x, tot, rc);
-        }
+    const T tot = total;
+    const double rc = sizeof(T) == 4 ? 1.0 / (double)tot : 0.0;
+    for (long s = threadIdx.x; s < S; s += SCALE_BLOCK) {
+        const T x = src[lay_at<LIN>(in, r + in.row0, s, S, blk)];
+        dst[lay_at<LOUT>(out, r + out.row0, s, S, blk)] = scale_q(x, tot, rc);
     }
 }
 
 template <typename T, int LIN, int LOUT>
-__global__ __launch_bounds__(SCALE_BLOCK) void scale_rows(kun_cs::View in, kun_cs::View out, long S, long rows,
-                                                           int blk) {
-    scale_block<T, LIN, LOUT, SCALE_ROWS>(in, out, S, rows, blk, (long)blockIdx.x * SCALE_ROWS, nullptr);
-}
-
-template <typename T, int LIN>
-__global__ __launch_bounds__(SCALE_BLOCK) void scale_sums(kun_cs::View in, long S, long rows, int blk, T *sums) {
-    scale_block<T, LIN, LIN, SCALE_SUM_ROWS>(in, in, S, rows, blk, (long)blockIdx.x * SCALE_SUM_ROWS, sums);
+__global__ __launch_bounds__(SCALE_BLOCK) void scale_rows(kun_cs::View in, kun_cs::View out, long S, int blk) {
+    scale_row<T, LIN, LOUT>(in, out, S, blk, blockIdx.x);
 }
 
 // out = x / sum of its row, or NaN where x == 0 and the sum is 0: workgroup
@@ -811,14 +917,13 @@ __global__ __launch_bounds__(256) void scale_div(kun_cs::View in, kun_cs::View o
 template <typename T> __global__ __launch_bounds__(SCALE_BLOCK) void scale_segs(const kun_cs::Seg *segs) {
     const kun_cs::Seg g = segs[blockIdx.x];
     const kun_cs::View in{const_cast<void *>(g.in), 2, 1, 0}, out{g.out, 2, 1, 0};
-    scale_block<T, 2, 2, SCALE_ROWS>(in, out, g.n, 1, 1, 0, nullptr);
+    scale_row<T, 2, 2>(in, out, g.n, 1, 0);
 }
 
 template <typename T, int LIN, int LOUT>
 hipError_t launch_scale_split(const kun_cs::View &in, const kun_cs::View &out, long S, long rows, int blk,
                               kun_cs::Sink &sink, T *sums) {
-    hipError_t e = sink_launch(sink, scale_sums<T, LIN>, dim3((unsigned)((rows + SCALE_SUM_ROWS - 1) / SCALE_SUM_ROWS)),
-                               dim3(SCALE_BLOCK), in, S, rows, blk, sums);
+    hipError_t e = sink_launch(sink, scale_sums<T, LIN>, dim3((unsigned)rows), dim3(64), in, S, rows, blk, sums);
     if (e != hipSuccess) return e;
     const long per = 256L * SCALE_DIV_ITEMS;
     return sink_launch(sink, scale_div<T, LIN, LOUT>,
@@ -834,12 +939,12 @@ hipError_t launch_scale_t(const kun_cs::View &in, const kun_cs::View &out, long 
         if (in.layout == 1 && out.layout == 1) return launch_scale_split<T, 1, 1>(in, out, S, rows, blk, sink, sums);
         return launch_scale_split<T, -1, -1>(in, out, S, rows, blk, sink, sums);
     }
-    const dim3 grid((unsigned)((rows + SCALE_ROWS - 1) / SCALE_ROWS));
+    const dim3 grid((unsigned)rows);
     if (in.layout == 1 && out.layout == 1)
-        return sink_launch(sink, scale_rows<T, 1, 1>, grid, dim3(SCALE_BLOCK), in, out, S, rows, blk);
+        return sink_launch(sink, scale_rows<T, 1, 1>, grid, dim3(SCALE_BLOCK), in, out, S, blk);
     if (in.layout == 2 && out.layout == 2)
-        return sink_launch(sink, scale_rows<T, 2, 2>, grid, dim3(SCALE_BLOCK), in, out, S, rows, blk);
-    return sink_launch(sink, scale_rows<T, -1, -1>, grid, dim3(SCALE_BLOCK), in, out, S, rows, blk);
+        return sink_launch(sink, scale_rows<T, 2, 2>, grid, dim3(SCALE_BLOCK), in, out, S, blk);
+    return sink_launch(sink, scale_rows<T, -1, -1>, grid, dim3(SCALE_BLOCK), in, out, S, blk);
 }
 
 template <typename T, int BLOCK, int ITEMS, int KIND>

@@ -1,0 +1,58 @@
+"""Scale and Rank row kernels at the sizes and on the rows where their
+tiles, binades and buckets end, against the oracle (bit for bit)."""
+import numpy as np
+import pytest
+
+from kunquant_amd.codegen.program import program_text
+from kunquant_amd.runner import KunRunner as kr
+from kunquant_amd.workloads import catalog
+from oracle.kun_oracle import OracleProgram
+from tests.helpers import assert_bit_exact
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def executor():
+    return kr.createMultiThreadExecutor(4)
+
+
+def _check(executor, module, a, b):
+    _, mod = catalog.load(module)
+    T, S = a.shape
+    ins = {"a": a, "b": b}
+    got = kr.runGraph(executor, mod, ins, 0, T)
+    exp = OracleProgram(program_text(catalog.module_ir(module))).run(ins, S, T, 0, T, nthreads=4)
+    for k in exp:
+        assert_bit_exact(got[k], exp[k], f"{module} {k} S={S}")
+
+
+def _sum_rows(S, dt, seed):
+    """Rows whose running sum of |x| meets ties, binades and limits."""
+    rng = np.random.default_rng(seed)
+    f = np.finfo(dt)
+    one = rng.integers(0, 1 << 20, S).astype(np.float64)
+    with np.errstate(all="ignore"):
+        rows = [
+            # every other cell is half a unit of the sum: the tie goes by the sum's last bit
+            np.concatenate([[1024.0], rng.integers(0, 4, max(0, S - 1)) * 512.0 * f.eps])[:S],
+            np.concatenate([[1024.0 * (1 + f.eps)], np.full(max(0, S - 1), 512.0 * f.eps)])[:S],
+            one * (1 if dt == np.float32 else 2.0 ** 26 + 0.5),          # whole numbers past the mantissa
+            2.0 ** (np.arange(S) % 60 - 30.0),                            # many binades, up and down
+            np.minimum(2.0 ** np.minimum(np.arange(S) / 5.0, 200.0), 1e30),
+            rng.integers(0, 1 << 12, S) * float(f.smallest_subnormal),    # subnormal sums, into the normal ones
+            np.full(S, float(f.max) / 3.0),                               # overflow to infinity
+            np.where(np.arange(S) == S // 3, np.inf, 1.0),
+            np.where(np.arange(S) % 7 == 0, np.nan, rng.standard_normal(S)),
+            np.zeros(S),
+            np.exp(rng.standard_normal(S) * 3.0),
+            rng.standard_normal(S),
+        ]
+    return np.ascontiguousarray(np.stack(rows).astype(dt))
+
+
+@pytest.mark.parametrize("module", ["cs_f32", "cs_f64"])
+@pytest.mark.parametrize("S", [1, 15, 17, 1023, 1024, 1025, 2049, 3071, 9000])
+def test_scale_sums_in_order(executor, module, S):
+    dt = catalog.load(module)[1].dtype
+    _check(executor, module, _sum_rows(S, dt, S), _sum_rows(S, dt, S + 1))

@@ -5,9 +5,10 @@
 // [lo, hi): sum = (lo + hi + 1) * (hi - lo) / 2 in integers, then
 // T(sum) / T(hi - lo) / T(n). -0 and +0 tie (std::sort / equal_range use
 // operator<). On the device a row's values become order-preserving integer
-// keys (-0 canonicalised to +0, NaN to the largest key) and are sorted with
-// their stocks by an LSD radix sort in LDS, 4-bit digits counted per lane
-// (CountRank, below); tie groups are read off the sorted order.
+// keys (-0 canonicalised to +0, NaN to the largest key) and are cut into
+// buckets of a key or two in LDS; a key's tie group is counted within its
+// bucket (BucketRank, below). Rows whose buckets stay crowded are sorted, by
+// an LSD radix sort with 4-bit digits counted per lane (CountRank).
 //
 // Scale (restates cpp/Kun/Scale.hpp:13-46): sum of |x| over non-NaN values
 // accumulated sequentially in stock order (bit-exact order), then
@@ -48,6 +49,15 @@ template <int LAY> __device__ __forceinline__ size_t lay_at(const kun_cs::View &
     if (LAY == 1) return (size_t)row * S + s;
     if (LAY == 2) return (size_t)s;
     return cs_at(v.layout, row, s, S, v.rows, blk);
+}
+
+// cell (row, s0 + i), s0 the same on every lane: for rows whose cells are
+// consecutive the address is a scalar one plus the lane's i, and no lane
+// keeps an index per cell
+template <int LAY, typename T>
+__device__ __forceinline__ T *cell_at(T *p, const kun_cs::View &v, long row, int s0, int i, long S, int blk) {
+    if (LAY == -1) return p + lay_at<LAY>(v, row, s0 + i, S, blk);
+    return p + lay_at<LAY>(v, row, s0, S, blk) + (unsigned)i;
 }
 
 // A kernel launch through a sink: the arguments converted to the kernel's
@@ -128,14 +138,19 @@ template <typename V> __device__ __forceinline__ V wave_or(V v) {
 }
 
 // rank of every member of the tie group at sorted positions [a, b) among n
-// non-NaN values
-template <typename T> __device__ __forceinline__ T group_rank(int a, int b, int n) {
+// non-NaN values; rn = RN(1 / n) in double
+template <typename T> __device__ __forceinline__ T group_rank(int a, int b, int n, double rn) {
     // rows of at most 16384 stocks: (a + b + 1) * (b - a) < 2^31, so the
     // reference's integer sum fits 32 bits and converts to T the same way
     const int32_t sum = (a + b + 1) * (b - a) / 2;
-    // x / 1 == x exactly: a group of one skips the first division
-    const T q = (b - a == 1) ? (T)sum : (T)sum / (T)(b - a);
-    return q / (T)n;
+    // where the sum converts exactly, its quotient by b - a is (a + b + 1) / 2
+    // exactly; only the largest tie groups of float rows need the division
+    T q = (T)(a + b + 1) * T(0.5);
+    if (sizeof(T) == 4 && sum >= 1 << 24) q = (T)sum / (T)(b - a);
+    // q >= 1, so the float quotient is normal and the double product exact
+    // (kun::div_rc)
+    if constexpr (sizeof(T) == 4) return kun::div_const(q, rn, (float)n);
+    else return q / (T)n;
 }
 
 // ---- Rank of long 64-bit rows: keys-only LSD radix sort -------------------
@@ -298,11 +313,12 @@ template <typename T, int BLOCK, int ITEMS> struct KeysRank {
         rank_by_search(sm, key, n, dst, out, S, blk, t, base);
     }
 
-    static __device__ __forceinline__ T rank_of(int a, int b, int n) { return group_rank<T>(a, b, n); }
+    static __device__ __forceinline__ T rank_of(int a, int b, int n, double rn) { return group_rank<T>(a, b, n, rn); }
 
     static __device__ __forceinline__ void rank_by_search(Smem &sm, const K (&mine)[ITEMS], int n, T *dst,
                                                           const kun_cs::View &out, long S, int blk, long t,
                                                           int base) {
+        const double rn = 1.0 / (double)n;
         // groups of G keys at a time, their searches interleaved
         constexpr int G = ITEMS < 4 ? ITEMS : 4;
 #pragma unroll
@@ -359,12 +375,27 @@ template <typename T, int BLOCK, int ITEMS> struct KeysRank {
             for (int j = 0; j < G; j++) {
                 const long s = base + (j0 + j) * 64;
                 if (s >= S) continue;
-                const T r = (mine[j0 + j] != ~K(0) && lo[j] < n) ? rank_of(lo[j], hi[j], n) : kun::qnan<T>();
+                const T r = (mine[j0 + j] != ~K(0) && lo[j] < n) ? rank_of(lo[j], hi[j], n, rn) : kun::qnan<T>();
                 dst[cs_at(out.layout, t + out.row0, s, S, out.rows, blk)] = r;
             }
         }
     }
 };
+
+__device__ __forceinline__ uint32_t lane_value(uint32_t v, int l) {
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, l);
+}
+__device__ __forceinline__ uint64_t lane_value(uint64_t v, int l) {
+    return (uint64_t)lane_value((uint32_t)(v >> 32), l) << 32 | lane_value((uint32_t)v, l);
+}
+
+// the value CTRL brings from a lane before this one, 0 where there is none
+template <int CTRL, int ROWS> __device__ __forceinline__ uint32_t dpp_before(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
+}
+template <int CTRL, int ROWS> __device__ __forceinline__ uint64_t dpp_before(uint64_t v) {
+    return (uint64_t)dpp_before<CTRL, ROWS>((uint32_t)(v >> 32)) << 32 | dpp_before<CTRL, ROWS>((uint32_t)v);
+}
 
 // inclusive prefix sum / max over the 64 lanes by DPP row shifts and row
 // broadcasts (rows of 16 lanes, then across rows); max assumes values >= 0
@@ -577,7 +608,7 @@ template <typename T, int BLOCK, int ITEMS> struct CountRank {
         ties<LOUT>(sm, key, id2, n, dst, out, S, blk, t);
     }
 
-    static __device__ __forceinline__ T rank_of(int a, int b, int n) { return group_rank<T>(a, b, n); }
+    static __device__ __forceinline__ T rank_of(int a, int b, int n, double rn) { return group_rank<T>(a, b, n, rn); }
 
     // sorted keys at positions P = tid*ITEMS + j (registers and sm.key)
     template <int LOUT>
@@ -616,9 +647,10 @@ template <typename T, int BLOCK, int ITEMS> struct CountRank {
             if (P < n && last[j]) endof[a[j]] = P + 1;
         }
         __syncthreads();
+        const double rn = 1.0 / (double)n;
         T r[ITEMS];
 #pragma unroll
-        for (int j = 0; j < ITEMS; j++) r[j] = P0 + j < n ? rank_of(a[j], endof[a[j]], n) : kun::qnan<T>();
+        for (int j = 0; j < ITEMS; j++) r[j] = P0 + j < n ? rank_of(a[j], endof[a[j]], n, rn) : kun::qnan<T>();
         __syncthreads();
         T *res = (T *)sm.key;
 #pragma unroll
@@ -631,36 +663,320 @@ template <typename T, int BLOCK, int ITEMS> struct CountRank {
     }
 };
 
-// KIND 0: CountRank (pairs); 1: KeysRank (64-bit keys beyond 8192 stocks)
-template <typename T, int BLOCK, int ITEMS, int KIND>
+// ---- Rank: buckets that follow the row's distribution ----------------------
+//
+// Ranks need no sorted order, only how many keys lie below each key and how
+// many equal it. The row is cut into buckets by a monotone map of the keys,
+// fine enough that a bucket holds a key or two whatever the distribution:
+//  1. a histogram of NC coarse buckets, the leading bits of key - smallest
+//     key;
+//  2. its prefix sum gives every coarse bucket as many position pairs as it
+//     has keys, split evenly over its range: position = 2 * first + (fraction
+//     within the bucket) * 2 * count. Within a coarse bucket (at most a
+//     fraction of an octave where the row spans several) values are near
+//     enough to evenly spread;
+//  3. a histogram over the positions (16-bit counts, two to a word); a key's
+//     turn in its bucket is the value its count had before it;
+//  4. the prefix sum of that histogram gives each bucket its place, and the
+//     keys are written there (sorted up to the order inside a bucket);
+//  5. every lane, which still holds the keys it loaded, counts the smaller
+//     and equal keys of each one's bucket, four at a time. Reading past a
+//     bucket's end is harmless: later buckets hold larger keys, and the keys
+//     end with four of the largest pattern.
+// Buckets of more than DEEP keys are whole tie groups as a rule (discrete
+// values): a lane whose key differs from its bucket's first one raises a
+// flag, and unless some bucket of the row is both deep and mixed, a deep
+// bucket's bounds are the tie group's. Returns false, with nothing written,
+// if the row has such a bucket; the caller then sorts it.
+//
+// 2 N positions (FSH = 0), or N / 2 (FSH = 2) where 64-bit keys leave less
+// LDS.
+//
+// 1024 rows of 8192 floats: 37 us a launch, 92 by the sort (floor 13 us at
+// the card's copy rate); 750 rows of 5003 doubles: 43 against 191, the sort
+// needing 16 passes; one row of 5000 doubles: 12 against 54; a pool cycle's
+// Rank segments of about 2200 stocks: 7.9 against 15. Bound by LDS accesses
+// and the instructions around them (about ten accesses a key, most of them
+// to random banks). Two workgroups a CU are worth 43 -> 37 us for float rows
+// of 8192 and take 64 registers, so values are packed and taken apart again
+// rather than kept.
+template <typename T, int BLOCK, int ITEMS, int FSH> struct BucketRank {
+    using K = typename KeyOf<T>::K;
+    static constexpr int N = BLOCK * ITEMS;
+    static constexpr int NW = BLOCK / 64;
+    static constexpr int NC = BLOCK * (FSH == 0 && ITEMS >= 4 ? ITEMS / 4 : 1);
+    static constexpr int CW = NC / BLOCK;          // coarse buckets per lane
+    static constexpr int FWORDS = N >> FSH;        // words of two positions
+    static constexpr int FW = FWORDS / BLOCK;      // of them per lane
+    static constexpr int DEEP = 64;
+    static_assert(FW >= 1 && N <= 16384, "positions and counts are 16-bit");
+    struct alignas(16) Smem {
+        uint32_t fine[FWORDS + 4]; // counts, then first places, of the positions 2w and 2w + 1
+        K key[N + 4];              // keys by bucket
+        uint32_t coarse[NC + 1];   // counts, then first keys
+        K wmax[NW], wmin[NW];
+        uint32_t wn[NW], wc[NW], wf[NW];
+        uint32_t mixed;
+    };
+
+    static __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+        v = max(v, dpp_before<0x111, 0xf>(v));
+        v = max(v, dpp_before<0x112, 0xf>(v));
+        v = max(v, dpp_before<0x114, 0xf>(v));
+        v = max(v, dpp_before<0x118, 0xf>(v));
+        v = max(v, dpp_before<0x142, 0xa>(v));
+        v = max(v, dpp_before<0x143, 0xc>(v));
+        return lane_value(v, 63);
+    }
+    static __device__ __forceinline__ uint64_t wave_max(uint64_t v) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            const uint64_t u = __shfl_xor(v, o, 64);
+            v = u > v ? u : v;
+        }
+        return v;
+    }
+    // sum of the wavefronts' totals before wavefront w
+    static __device__ __forceinline__ uint32_t before(const uint32_t (&tot)[NW], int w, int lane) {
+        const uint32_t p = dpp_row_incl_sum(lane < NW ? tot[lane] : 0u);
+        return w ? lane_value(p, w - 1) : 0u;
+    }
+
+    template <int LIN, int LOUT>
+    static __device__ __forceinline__ bool row(Smem &sm, const kun_cs::View &in, const kun_cs::View &out, long S,
+                                               int blk, long t) {
+        const int tid = threadIdx.x, lane = tid & 63;
+        const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+        const T *src = (const T *)in.ptr;
+        T *dst = (T *)out.ptr;
+        const long rin = t + in.row0;
+        const int n_all = (int)S;
+        T xs[ITEMS];
+#pragma unroll
+        for (int j = 0; j < ITEMS; j++) {
+            const int left = n_all - j * BLOCK;
+            if (left > 0) xs[j] = *cell_at<LIN>(src, in, rin, j * BLOCK, min(tid, left - 1), S, blk);
+        }
+#pragma unroll
+        for (int i = 0; i < CW; i++) sm.coarse[i * BLOCK + tid] = 0;
+#pragma unroll
+        for (int i = 0; i < FW; i++) sm.fine[i * BLOCK + tid] = 0;
+        if (tid == 0) sm.mixed = 0;
+        K key[ITEMS]; // ~0: missing
+        K kmax = 0, kinv = 0;
+        uint32_t n = 0;
+#pragma unroll
+        for (int j = 0; j < ITEMS; j++) {
+            key[j] = tid < n_all - j * BLOCK ? rank_key(xs[j]) : ~K(0);
+            const bool live = key[j] != ~K(0);
+            n += (uint32_t)__popcll(__ballot(live));
+            const K a = live ? key[j] : K(0), b = ~key[j];
+            kmax = a > kmax ? a : kmax;
+            kinv = b > kinv ? b : kinv; // a missing cell's is 0
+        }
+        kmax = wave_max(kmax);
+        kinv = wave_max(kinv);
+        if (lane == 0) {
+            sm.wmax[w] = kmax;
+            sm.wmin[w] = kinv;
+            sm.wn[w] = n;
+        }
+        __syncthreads();
+        // lane q < NW holds wavefront q's
+        n = lane_value(dpp_row_incl_sum(lane < NW ? sm.wn[lane] : 0u), NW - 1);
+        kmax = wave_max(lane < NW ? sm.wmax[lane] : K(0));
+        kinv = wave_max(lane < NW ? sm.wmin[lane] : K(0));
+        const K kmin = ~kinv;
+        int sh = 0; // bits of key - kmin below the coarse bucket's
+        if (n && kmax != kmin) {
+            const K range = kmax - kmin;
+            const int bits = sizeof(K) == 8 ? 64 - __builtin_clzll((uint64_t)range) : 32 - __builtin_clz((uint32_t)range);
+            constexpr int CB = __builtin_ctz(NC);
+            sh = bits > CB ? bits - CB : 0;
+        }
+        sh = __builtin_amdgcn_readfirstlane(sh);
+        // Missing cells go through the same instructions, adding nothing to a
+        // count of their lane's own and storing the largest pattern where the
+        // keys end with it anyway: no branch per cell.
+        // 1. coarse counts
+#pragma unroll
+        for (int j = 0; j < ITEMS; j++) {
+            const bool live = key[j] != ~K(0);
+            atomicAdd(&sm.coarse[live ? (uint32_t)((key[j] - kmin) >> sh) : (uint32_t)tid], live ? 1u : 0u);
+        }
+        __syncthreads();
+        // 2. first keys of the coarse buckets
+        {
+            uint32_t c[CW], s = 0;
+#pragma unroll
+            for (int i = 0; i < CW; i++) {
+                c[i] = sm.coarse[tid * CW + i];
+                s += c[i];
+            }
+            const uint32_t incl = dpp_incl_sum(s);
+            if (lane == 63) sm.wc[w] = incl;
+            __syncthreads();
+            uint32_t run = before(sm.wc, w, lane) + incl - s;
+#pragma unroll
+            for (int i = 0; i < CW; i++) {
+                sm.coarse[tid * CW + i] = run;
+                run += c[i];
+            }
+            if (tid == 0) sm.coarse[NC] = n;
+        }
+        __syncthreads();
+        // 3. positions, and each key's turn in its bucket
+        uint32_t at[ITEMS]; // position, turn in the high half
+#pragma unroll
+        for (int j = 0; j < ITEMS; j++) {
+            const K r = key[j] != ~K(0) ? key[j] - kmin : K(0);
+            const uint32_t b = (uint32_t)(r >> sh);
+            const uint32_t c0 = sm.coarse[b], c1 = sm.coarse[b + 1];
+            // the bits below the bucket's, as a 32-bit fraction of its range
+            constexpr int TOP = (int)sizeof(K) * 8 - 1;
+            const uint32_t frac = (uint32_t)(((r << 1) << (TOP - sh)) >> (TOP - 31));
+            at[j] = (2 * c0 + __umulhi(frac, 2 * (c1 - c0))) >> FSH;
+        }
+#pragma unroll
+        for (int j = 0; j < ITEMS; j++) {
+            const bool live = key[j] != ~K(0);
+            at[j] = live ? at[j] : 2u * (uint32_t)tid;
+            const uint32_t half = (at[j] & 1) * 16;
+            const uint32_t old = atomicAdd(&sm.fine[at[j] >> 1], (live ? 1u : 0u) << half);
+            at[j] |= (old >> half) << 16;
+            // one register a key from here on, not the three it is made of
+            asm volatile("" : "+v"(at[j]));
+        }
+        __syncthreads();
+        // 4. first places of the buckets
+        {
+            uint32_t c[FW], s = 0;
+#pragma unroll
+            for (int i = 0; i < FW; i++) {
+                c[i] = sm.fine[tid * FW + i];
+                s += (c[i] & 0xffffu) + (c[i] >> 16);
+            }
+            const uint32_t incl = dpp_incl_sum(s);
+            if (lane == 63) sm.wf[w] = incl;
+            __syncthreads();
+            uint32_t run = before(sm.wf, w, lane) + incl - s;
+#pragma unroll
+            for (int i = 0; i < FW; i++) {
+                const uint32_t mid = run + (c[i] & 0xffffu);
+                sm.fine[tid * FW + i] = run | mid << 16;
+                run = mid + (c[i] >> 16);
+            }
+            if (tid == 0) sm.fine[FWORDS] = n;
+            if (tid < 4) sm.key[n + tid] = ~K(0);
+        }
+        __syncthreads();
+        uint32_t span[ITEMS]; // first place of the bucket, end in the high half
+#pragma unroll
+        for (int j = 0; j < ITEMS; j++) {
+            const uint32_t p = at[j] & 0xffffu;
+            span[j] = __builtin_amdgcn_alignbit(sm.fine[(p >> 1) + 1], sm.fine[p >> 1], (p & 1) * 16);
+            sm.key[key[j] != ~K(0) ? (span[j] & 0xffffu) + (at[j] >> 16) : n] = key[j];
+            asm volatile("" : "+v"(span[j]));
+        }
+        __syncthreads();
+        // 5. deep buckets must be tie groups
+        auto size = [&](int j) { return (int)(span[j] >> 16) - (int)(span[j] & 0xffffu); };
+        bool deep = false;
+#pragma unroll
+        for (int j = 0; j < ITEMS; j++) deep = deep || (key[j] != ~K(0) && size(j) > DEEP);
+        if (__ballot(deep)) {
+            bool mixed = false;
+#pragma unroll
+            for (int j = 0; j < ITEMS; j++) asm volatile("" : "+v"(span[j]));
+#pragma unroll
+            for (int j = 0; j < ITEMS; j++)
+                if (key[j] != ~K(0) && size(j) > DEEP) mixed = mixed || sm.key[span[j] & 0xffffu] != key[j];
+            if (__ballot(mixed) && lane == 0) sm.mixed = 1;
+        }
+        __syncthreads();
+        if (__builtin_amdgcn_readfirstlane((int)sm.mixed)) return false; // the same on every lane
+        const double rn = 1.0 / (double)(int)n;
+        constexpr int G = ITEMS < 16 / (int)sizeof(K) ? ITEMS : 16 / (int)sizeof(K); // keys counted side by side
+#pragma unroll
+        for (int j0 = 0; j0 < ITEMS; j0 += G) {
+            K q[G][4];
+            int lt[G], le[G];
+            // bounds and sizes taken from the packed word again for every
+            // group, rather than kept for all keys at once
+#pragma unroll
+            for (int g = 0; g < G; g++) asm volatile("" : "+v"(span[j0 + g]));
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int g = 0; g < G; g++)
+#pragma unroll
+                for (int u = 0; u < 4; u++) q[g][u] = sm.key[(span[j0 + g] & 0xffffu) + u];
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                lt[g] = le[g] = 0;
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    lt[g] += q[g][u] < key[j0 + g] ? 1 : 0;
+                    le[g] += q[g][u] <= key[j0 + g] ? 1 : 0;
+                }
+            }
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                const int j = j0 + g, sz = size(j);
+                const bool live = key[j] != ~K(0);
+                const int a = (int)(span[j] & 0xffffu);
+                if (live && sz > 4 && sz <= DEEP)
+                    for (int i = a + 4; i < a + sz; i++) {
+                        const K k = sm.key[i];
+                        lt[g] += k < key[j] ? 1 : 0;
+                        le[g] += k <= key[j] ? 1 : 0;
+                    }
+                if (sz > DEEP) le[g] = sz;
+                const T r = live ? group_rank<T>(a + lt[g], a + le[g], (int)n, rn) : kun::qnan<T>();
+                if (tid < n_all - j * BLOCK) *cell_at<LOUT>(dst, out, t + out.row0, j * BLOCK, tid, S, blk) = r;
+            }
+        }
+        return true;
+    }
+};
+
+// KIND 0: CountRank (pairs); 1: KeysRank (64-bit keys beyond 8192 stocks):
+// how a row is sorted whose buckets are deep and mixed. LAY: both views'
+// layout (-1: read from the views)
+template <typename T, int BLOCK, int ITEMS, int KIND, int LAY>
 __device__ __forceinline__ void rank_row_k(const kun_cs::View &in, const kun_cs::View &out, long S, int blk,
                                            const long t) {
-    if constexpr (KIND == 0) {
-        using R = CountRank<T, BLOCK, ITEMS>;
-        __shared__ typename R::Smem sm;
-        // rows of TS buffers (every batch run's temporaries) with their
-        // addressing fixed at compile time; other layouts read the view's
-        if (in.layout == 1 && out.layout == 1) R::template row<1, 1>(sm, in, out, S, blk, t);
-        else R::template row<-1, -1>(sm, in, out, S, blk, t);
-    } else {
-        using R = KeysRank<T, BLOCK, ITEMS>;
-        __shared__ typename R::Smem sm;
-        R::row(sm, in, out, S, blk, t);
-    }
+    if (S <= 0) return; // uniform: nothing to rank
+    using B = BucketRank<T, BLOCK, ITEMS, KIND == 0 ? 0 : 2>;
+    using R = std::conditional_t<KIND == 0, CountRank<T, BLOCK, ITEMS>, KeysRank<T, BLOCK, ITEMS>>;
+    __shared__ union Smem {
+        typename B::Smem b;
+        typename R::Smem r;
+        __device__ Smem() {}
+    } sm;
+    if (B::template row<LAY, LAY>(sm.b, in, out, S, blk, t)) return;
+    __syncthreads(); // the flag's readers are done with the shared memory
+    if constexpr (KIND == 0) R::template row<LAY, LAY>(sm.r, in, out, S, blk, t);
+    else R::row(sm.r, in, out, S, blk, t);
+}
+
+// Wavefronts per SIMD the registers leave room for: two workgroups of 1024
+// lanes share a CU where their LDS allows it (float rows up to 8192)
+template <typename T, int BLOCK, int ITEMS> constexpr int rank_waves() {
+    return BLOCK * ITEMS * (int)sizeof(T) <= 32768 ? 8 : 4;
 }
 
 // one workgroup per row of the views
-template <typename T, int BLOCK, int ITEMS, int KIND>
-__global__ __launch_bounds__(BLOCK) void rank_rows(kun_cs::View in, kun_cs::View out, long S, int blk) {
-    rank_row_k<T, BLOCK, ITEMS, KIND>(in, out, S, blk, blockIdx.x);
+template <typename T, int BLOCK, int ITEMS, int KIND, int LAY>
+__global__ __launch_bounds__(BLOCK, (rank_waves<T, BLOCK, ITEMS>())) void rank_rows(kun_cs::View in, kun_cs::View out, long S, int blk) {
+    rank_row_k<T, BLOCK, ITEMS, KIND, LAY>(in, out, S, blk, blockIdx.x);
 }
 
 // one workgroup per segment (a contiguous run of stocks of one row)
 template <typename T, int BLOCK, int ITEMS, int KIND>
-__global__ __launch_bounds__(BLOCK) void rank_segs(const kun_cs::Seg *segs) {
+__global__ __launch_bounds__(BLOCK, (rank_waves<T, BLOCK, ITEMS>())) void rank_segs(const kun_cs::Seg *segs) {
     const kun_cs::Seg g = segs[blockIdx.x];
     const kun_cs::View in{const_cast<void *>(g.in), 2, 1, 0}, out{g.out, 2, 1, 0};
-    rank_row_k<T, BLOCK, ITEMS, KIND>(in, out, g.n, 1, 0);
+    rank_row_k<T, BLOCK, ITEMS, KIND, 2>(in, out, g.n, 1, 0);
 }
 
 // ---- Scale: row sums in stock order, a tile at a time ---------------------
@@ -693,21 +1009,6 @@ __global__ __launch_bounds__(BLOCK) void rank_segs(const kun_cs::Seg *segs) {
 // against 24.5.
 constexpr int CHAIN_K = 16;
 constexpr int CHAIN_TILE = 64 * CHAIN_K;
-
-__device__ __forceinline__ uint32_t lane_value(uint32_t v, int l) {
-    return (uint32_t)__builtin_amdgcn_readlane((int)v, l);
-}
-__device__ __forceinline__ uint64_t lane_value(uint64_t v, int l) {
-    return (uint64_t)lane_value((uint32_t)(v >> 32), l) << 32 | lane_value((uint32_t)v, l);
-}
-
-// the value CTRL brings from a lane before this one, 0 where there is none
-template <int CTRL, int ROWS> __device__ __forceinline__ uint32_t dpp_before(uint32_t v) {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
-}
-template <int CTRL, int ROWS> __device__ __forceinline__ uint64_t dpp_before(uint64_t v) {
-    return (uint64_t)dpp_before<CTRL, ROWS>((uint32_t)(v >> 32)) << 32 | dpp_before<CTRL, ROWS>((uint32_t)v);
-}
 
 // inclusive scan over the lanes of the runs' moves from an even (i0) and an
 // odd (i1) sum, in units
@@ -950,7 +1251,14 @@ hipError_t launch_scale_t(const kun_cs::View &in, const kun_cs::View &out, long 
 template <typename T, int BLOCK, int ITEMS, int KIND>
 hipError_t launch_rank_n(const kun_cs::View &in, const kun_cs::View &out, long S, long rows, int blk,
                          kun_cs::Sink &sink) {
-    return sink_launch(sink, rank_rows<T, BLOCK, ITEMS, KIND>, dim3((unsigned)rows), dim3(BLOCK), in, out, S, blk);
+    // rows of TS buffers (every batch run's temporaries) and single rows with
+    // their addressing fixed at compile time; other layouts read the views'
+    const dim3 grid((unsigned)rows), block(BLOCK);
+    if (in.layout == 1 && out.layout == 1)
+        return sink_launch(sink, rank_rows<T, BLOCK, ITEMS, KIND, 1>, grid, block, in, out, S, blk);
+    if (in.layout == 2 && out.layout == 2)
+        return sink_launch(sink, rank_rows<T, BLOCK, ITEMS, KIND, 2>, grid, block, in, out, S, blk);
+    return sink_launch(sink, rank_rows<T, BLOCK, ITEMS, KIND, -1>, grid, block, in, out, S, blk);
 }
 
 // Workgroup shape by row length: at most 1024 lanes, up to 16 keys per lane;

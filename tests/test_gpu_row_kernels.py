@@ -56,3 +56,37 @@ def _sum_rows(S, dt, seed):
 def test_scale_sums_in_order(executor, module, S):
     dt = catalog.load(module)[1].dtype
     _check(executor, module, _sum_rows(S, dt, S), _sum_rows(S, dt, S + 1))
+
+
+def _rank_rows(S, dt, seed):
+    """Rows whose buckets are empty, deep, mixed, or at the ends of the key range."""
+    rng = np.random.default_rng(seed)
+    f = np.finfo(dt)
+    i = np.arange(S)
+    with np.errstate(all="ignore"):
+        rows = [
+            rng.standard_normal(S),
+            100.0 * np.exp(rng.standard_normal(S) * 0.6),
+            rng.integers(0, 10, S).astype(np.float64),                            # deep tie groups
+            np.where(i % 2 == 0, 0.0, rng.random(S)),                             # half of them zero
+            np.where(i % 2 == 0, 100.0 * (1 + (i % 97) * float(f.eps)), 50.0 + 150.0 * rng.random(S)),  # deep and mixed
+            np.where(i == S // 2, -float(f.max), rng.random(S)),                  # one outlier
+            np.where(i % 3 == 0, np.inf, np.where(i % 3 == 1, -np.inf, rng.standard_normal(S))),
+            np.where(i % 2 == 0, np.nan, -rng.random(S)),
+            np.full(S, 7.5),
+            np.where(i == 0, 1.0, np.nan),
+            np.full(S, np.nan),
+            rng.integers(-50, 50, S) * float(f.smallest_subnormal),
+            rng.standard_normal(S) * 10.0 ** rng.uniform(-30, 30, S),
+            1.0 + rng.integers(0, 4 * S, S) * float(f.eps),                       # dense: neighbouring values
+            np.sort(rng.standard_normal(S)),
+            np.where(rng.random(S) < 0.5, -0.0, 0.0) + np.where(i % 5 == 0, rng.standard_normal(S), 0.0),
+        ]
+    return np.ascontiguousarray(np.stack(rows).astype(dt))
+
+
+@pytest.mark.parametrize("module", ["cs_f32", "cs_f64"])
+@pytest.mark.parametrize("S", [1, 2, 255, 256, 257, 513, 1025, 2048, 2049, 4097, 8191, 8193, 16383])
+def test_rank_buckets(executor, module, S):
+    dt = catalog.load(module)[1].dtype
+    _check(executor, module, _rank_rows(S, dt, S), _rank_rows(S, dt, S + 1)[::-1].copy())

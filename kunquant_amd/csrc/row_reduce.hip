@@ -7,9 +7,8 @@
 // stocks in stock order of x, y, x*x, y*y and x*y (no NaN skipping), each
 // divided by the stock count, then (XY - X*Y) / (sqrt(X2 - X*X) *
 // sqrt(Y2 - Y*Y)). The five sums are sequential chains in stock order (bit
-// parity); one lane owns one row and walks its stocks, the five chains
-// interleaved, loads issued a group of stocks ahead. With rank inputs, x is
-// the row's rank, computed by the Rank row kernel first.
+// parity). With rank inputs, x is the row's rank, computed by the Rank row
+// kernel first.
 //
 // aggregrate restates cpp/Kun/Aggregration.cpp:11-105: one lane per stock
 // walks the rows in order; a change of label closes a group and stores its
@@ -22,52 +21,119 @@
 
 namespace {
 
-constexpr int CORR_UNROLL = 8;
-
 __device__ __forceinline__ size_t rr_at(int sts, long t, long s, long S, long T, int blk) {
     return sts ? ((size_t)(s / blk) * T + t) * blk + s % blk : (size_t)t * S + s;
 }
 
-// rows [start, start + L) of x (layout `xsts`, rows of T) and y (`ysts`);
-// x may instead be a [L][S] TS array of ranks (xrows = L, xrow0 = 0)
-__global__ __launch_bounds__(64) void corr_rows(const float *x, int xsts, long xT, long xrow0, const float *y,
-                                                int ysts, long yT, float *out, long S, long start, long L, int blk) {
-    const long r = (long)blockIdx.x * 64 + threadIdx.x;
-    if (r >= L) return;
-    const long tx = r + xrow0, ty = r + start;
-    float XY = 0.f, X = 0.f, Y = 0.f, X2 = 0.f, Y2 = 0.f;
-    long s = 0;
-    for (; s + CORR_UNROLL <= S; s += CORR_UNROLL) {
-        float a[CORR_UNROLL], b[CORR_UNROLL];
+// Bound by the chains' latency: an add that waits for the one before it
+// takes 8.9 clocks, 5000 stocks 19 us, however little of the GPU they fill.
+// So each lane of a workgroup's first wavefront runs one chain of one row
+// (CORR_ROWS rows x 5 chains) and does nothing but read the next terms and
+// add; the other wavefronts load the rows a tile ahead and leave the terms --
+// a, b, a*a, b*b, a*b, each rounded as the chain would -- in LDS; and the
+// inputs of a call share a launch, so that their chains run side by side.
+// Rows are padded with -0, which leaves every sum as it is.
+//
+// 4 inputs of 1000 rows of 5000 stocks: 39 us; a lane that walked all five
+// chains of its own row, a launch per input, took 1910.
+constexpr int CORR_ROWS = 8, CORR_TILE = 128, CORR_STAGE = 256, CORR_CHAINS = 5;
+constexpr int CORR_BLOCK = 64 + CORR_STAGE;
+constexpr int CORR_STRIDE = CORR_TILE + 4; // chains of 16-byte reads start four banks apart
+constexpr int CORR_STEP = 16;              // terms read ahead of their adds
+constexpr int CORR_INPUTS = 16;            // inputs of one launch
+
+// rows [start, start + L) of the inputs (layout `xsts`, rows of T) and y
+// (`ysts`); x may instead be [L][S] TS arrays of ranks (xrows = L, xrow0 = 0)
+struct CorrArgs {
+    const float *x[CORR_INPUTS], *y;
+    float *out[CORR_INPUTS];
+    int xsts, ysts, blk;
+    long xT, xrow0, yT, S, start, L;
+};
+
+__global__ __launch_bounds__(CORR_BLOCK) void corr_rows(const CorrArgs A) {
+    __shared__ __attribute__((aligned(16))) float term[2][CORR_CHAINS * CORR_ROWS * CORR_STRIDE];
+    __shared__ float total[CORR_CHAINS][CORR_ROWS];
+    const float *x = A.x[blockIdx.y];
+    const long r0 = (long)blockIdx.x * CORR_ROWS;
+    const int nr = (int)(A.L - r0 < CORR_ROWS ? A.L - r0 : CORR_ROWS);
+    const int ntile = (int)((A.S + CORR_TILE - 1) / CORR_TILE);
+    constexpr int PER = CORR_ROWS * CORR_TILE / CORR_STAGE;
+    if (threadIdx.x >= 64) {
+        const int id = threadIdx.x - 64;
+        float a[PER], b[PER];
+        auto load = [&](int tile) {
 #pragma unroll
-        for (int k = 0; k < CORR_UNROLL; k++) {
-            a[k] = x[rr_at(xsts, tx, s + k, S, xT, blk)];
-            b[k] = y[rr_at(ysts, ty, s + k, S, yT, blk)];
-        }
+            for (int q = 0; q < PER; q++) {
+                const int e = id + q * CORR_STAGE, r = e / CORR_TILE;
+                const long s = (long)tile * CORR_TILE + e % CORR_TILE;
+                a[q] = b[q] = -0.f;
+                if (r < nr && s < A.S) {
+                    a[q] = x[rr_at(A.xsts, r0 + r + A.xrow0, s, A.S, A.xT, A.blk)];
+                    b[q] = A.y[rr_at(A.ysts, r0 + r + A.start, s, A.S, A.yT, A.blk)];
+                }
+            }
+        };
+        auto store = [&](int tile) {
+            float *t = term[tile & 1];
 #pragma unroll
-        for (int k = 0; k < CORR_UNROLL; k++) {
-            X = X + a[k];
-            Y = Y + b[k];
-            X2 = X2 + a[k] * a[k];
-            Y2 = Y2 + b[k] * b[k];
-            XY = XY + a[k] * b[k];
+            for (int q = 0; q < PER; q++) {
+                const int e = id + q * CORR_STAGE;
+                const bool in = (long)tile * CORR_TILE + e % CORR_TILE < A.S;
+                float *at = t + e / CORR_TILE * CORR_STRIDE + e % CORR_TILE;
+                constexpr int C = CORR_ROWS * CORR_STRIDE;
+                at[0] = a[q];
+                at[C] = b[q];
+                at[2 * C] = in ? a[q] * a[q] : -0.f; // (-0) * (-0) is +0
+                at[3 * C] = in ? b[q] * b[q] : -0.f;
+                at[4 * C] = in ? a[q] * b[q] : -0.f;
+            }
+        };
+        load(0);
+        store(0);
+        load(1);
+        for (int t = 0; t < ntile; t++) {
+            __syncthreads(); // tile t is stored, tile t - 1 summed
+            if (t + 1 < ntile) {
+                store(t + 1);
+                load(t + 2);
+            }
         }
+    } else {
+        const int chain = threadIdx.x / CORR_ROWS, r = threadIdx.x % CORR_ROWS;
+        const int at = (chain < CORR_CHAINS ? chain : 0) * CORR_ROWS * CORR_STRIDE + r * CORR_STRIDE;
+        float sum = 0.f;
+        for (int t = 0; t < ntile; t++) {
+            __syncthreads();
+            const float *v = term[t & 1] + at;
+            float g[CORR_STEP], h[CORR_STEP];
+#pragma unroll
+            for (int u = 0; u < CORR_STEP; u++) g[u] = v[u];
+#pragma unroll
+            for (int k = 0; k < CORR_TILE; k += 2 * CORR_STEP) {
+#pragma unroll
+                for (int u = 0; u < CORR_STEP; u++) h[u] = v[k + CORR_STEP + u];
+                __builtin_amdgcn_sched_barrier(0); // the reads stay ahead of the adds
+#pragma unroll
+                for (int u = 0; u < CORR_STEP; u++) sum = sum + g[u];
+                if (k + 2 * CORR_STEP < CORR_TILE)
+#pragma unroll
+                    for (int u = 0; u < CORR_STEP; u++) g[u] = v[k + 2 * CORR_STEP + u];
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = 0; u < CORR_STEP; u++) sum = sum + h[u];
+            }
+        }
+        if (chain < CORR_CHAINS) total[chain][r] = sum;
     }
-    for (; s < S; s++) {
-        const float a = x[rr_at(xsts, tx, s, S, xT, blk)], b = y[rr_at(ysts, ty, s, S, yT, blk)];
-        X = X + a;
-        Y = Y + b;
-        X2 = X2 + a * a;
-        Y2 = Y2 + b * b;
-        XY = XY + a * b;
+    __syncthreads();
+    if ((int)threadIdx.x < nr) {
+        const float n = (float)A.S;
+        const int r = threadIdx.x;
+        const float X = total[0][r] / n, Y = total[1][r] / n, X2 = total[2][r] / n, Y2 = total[3][r] / n;
+        const float XY = total[4][r] / n;
+        A.out[blockIdx.y][r0 + r] = (XY - X * Y) / (sqrtf(X2 - X * X) * sqrtf(Y2 - Y * Y));
     }
-    const float n = (float)S;
-    XY = XY / n;
-    X = X / n;
-    Y = Y / n;
-    X2 = X2 / n;
-    Y2 = Y2 / n;
-    out[r] = (XY - X * Y) / (sqrtf(X2 - X * X) * sqrtf(Y2 - Y * Y));
 }
 
 struct AggOut {
@@ -120,11 +186,29 @@ __global__ __launch_bounds__(64) void aggregate_cols(const T *in, const T *label
 
 namespace kun_cs {
 
-hipError_t launch_corr(const float *x, int xsts, long xT, long xrow0, const float *y, int ysts, long yT, float *out,
-                       long S, long start, long L, int blk, hipStream_t st) {
-    if (L <= 0) return hipSuccess;
-    hipLaunchKernelGGL(corr_rows, dim3((unsigned)((L + 63) / 64)), dim3(64), 0, st, x, xsts, xT, xrow0, y, ysts, yT,
-                       out, S, start, L, blk);
+int corr_inputs() { return CORR_INPUTS; }
+
+hipError_t launch_corr(int n, const float *const *x, int xsts, long xT, long xrow0, const float *y, int ysts, long yT,
+                       float *const *out, long S, long start, long L, int blk, hipStream_t st) {
+    if (L <= 0 || n <= 0) return hipSuccess;
+    if (n > CORR_INPUTS) return hipErrorInvalidValue;
+    CorrArgs a;
+    for (int i = 0; i < CORR_INPUTS; i++) {
+        a.x[i] = x[i < n ? i : 0];
+        a.out[i] = out[i < n ? i : 0];
+    }
+    a.y = y;
+    a.xsts = xsts;
+    a.ysts = ysts;
+    a.blk = blk;
+    a.xT = xT;
+    a.xrow0 = xrow0;
+    a.yT = yT;
+    a.S = S;
+    a.start = start;
+    a.L = L;
+    hipLaunchKernelGGL(corr_rows, dim3((unsigned)((L + CORR_ROWS - 1) / CORR_ROWS), (unsigned)n), dim3(CORR_BLOCK), 0,
+                       st, a);
     return hipGetLastError();
 }
 
@@ -148,6 +232,8 @@ hipError_t launch_aggregate(int dtype, const void *in, const void *labels, void 
 // ---- host drivers -----------------------------------------------------------
 #include <string.h>
 
+#include <algorithm>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -189,42 +275,59 @@ void corr_with(Executor &ex, bool device, int sts, bool rank_inputs, int n, cons
     HIPCHECK(hipSetDevice(ex.device));
     if (!st) st = ex.stream;
     const size_t in_bytes = (sts ? (S + blk - 1) / blk * blk : S) * T * sizeof(float);
-    std::unique_ptr<DevBuf> dtarget, dx, dout;
+    // a launch takes a group of inputs: as many as it can, and device copies
+    // and ranks together within a gigabyte
+    const size_t out_bytes = L * sizeof(float) + 4, rank_bytes = S * L * sizeof(float) + 4;
+    const size_t each = (device ? 0 : in_bytes + out_bytes) + (rank_inputs ? rank_bytes : 0);
+    const size_t fit = each ? std::max<size_t>(1, ((size_t)1 << 30) / each) : (size_t)kun_cs::corr_inputs();
+    const int group = (int)std::min<size_t>(std::min<size_t>(fit, (size_t)kun_cs::corr_inputs()), (size_t)n);
+    std::unique_ptr<DevBuf> dtarget;
+    std::vector<std::unique_ptr<DevBuf>> dx, dout, ranks;
     const float *y = target;
     if (!device) {
         dtarget.reset(new DevBuf(ex, in_bytes));
         HIPCHECK(hipMemcpyAsync(dtarget->p, target, in_bytes, hipMemcpyHostToDevice, st));
         y = (const float *)dtarget->p;
-        dx.reset(new DevBuf(ex, in_bytes));
-        dout.reset(new DevBuf(ex, L * sizeof(float) + 4));
     }
-    std::unique_ptr<DevBuf> ranks;
-    if (rank_inputs) ranks.reset(new DevBuf(ex, S * L * sizeof(float) + 4));
-    for (int i = 0; i < n; i++) {
-        const float *x = inputs[i];
-        float *o = outs[i];
+    for (int k = 0; k < group; k++) {
         if (!device) {
-            HIPCHECK(hipMemcpyAsync(dx->p, x, in_bytes, hipMemcpyHostToDevice, st));
-            x = (const float *)dx->p;
-            o = (float *)dout->p;
+            dx.emplace_back(new DevBuf(ex, in_bytes));
+            dout.emplace_back(new DevBuf(ex, out_bytes));
         }
-        hipError_t e;
-        if (rank_inputs) {
-            kun_cs::View vi{(void *)x, sts ? 0 : 1, (long)T, (long)start}, vo{ranks->p, 1, (long)L, 0};
-            e = kun_cs::launch_rank(0, vi, vo, (long)S, (long)L, blk, st);
-            if (e == hipSuccess)
-                e = kun_cs::launch_corr((const float *)ranks->p, 0, (long)L, 0, y, sts, (long)T, o, (long)S,
-                                        (long)start, (long)L, blk, st);
-        } else {
-            e = kun_cs::launch_corr(x, sts, (long)T, (long)start, y, sts, (long)T, o, (long)S, (long)start, (long)L,
-                                    blk, st);
+        if (rank_inputs) ranks.emplace_back(new DevBuf(ex, rank_bytes));
+    }
+    for (int i0 = 0; i0 < n; i0 += group) {
+        const int m = std::min(group, n - i0);
+        std::vector<const float *> x(m);
+        std::vector<float *> o(m);
+        hipError_t e = hipSuccess;
+        for (int k = 0; k < m; k++) {
+            x[k] = inputs[i0 + k];
+            o[k] = outs[i0 + k];
+            if (!device) {
+                HIPCHECK(hipMemcpyAsync(dx[k]->p, x[k], in_bytes, hipMemcpyHostToDevice, st));
+                x[k] = (const float *)dx[k]->p;
+                o[k] = (float *)dout[k]->p;
+            }
+            if (rank_inputs && e == hipSuccess) {
+                kun_cs::View vi{(void *)x[k], sts ? 0 : 1, (long)T, (long)start}, vo{ranks[k]->p, 1, (long)L, 0};
+                e = kun_cs::launch_rank(0, vi, vo, (long)S, (long)L, blk, st);
+                x[k] = (const float *)ranks[k]->p;
+            }
         }
+        if (e == hipSuccess)
+            e = rank_inputs ? kun_cs::launch_corr(m, x.data(), 0, (long)L, 0, y, sts, (long)T, o.data(), (long)S,
+                                                  (long)start, (long)L, blk, st)
+                            : kun_cs::launch_corr(m, x.data(), sts, (long)T, (long)start, y, sts, (long)T, o.data(),
+                                                  (long)S, (long)start, (long)L, blk, st);
         if (e != hipSuccess) throw Error(std::string("corrWith kernel: ") + hipGetErrorString(e));
-        if (!device) HIPCHECK(hipMemcpyAsync(outs[i], o, L * sizeof(float), hipMemcpyDeviceToHost, st));
+        if (!device)
+            for (int k = 0; k < m; k++)
+                HIPCHECK(hipMemcpyAsync(outs[i0 + k], o[k], L * sizeof(float), hipMemcpyDeviceToHost, st));
     }
     // host buffers are copied back; pooled scratch returns to the pool only
     // once the kernels reading it are done
-    if (!device || ranks) HIPCHECK(hipStreamSynchronize(st));
+    if (!device || rank_inputs) HIPCHECK(hipStreamSynchronize(st));
 }
 
 void aggregate(Executor &ex, bool device, int n, const void *const *inputs, const void *const *labels, int dtype,

@@ -6,6 +6,7 @@ import pytest
 from kunquant_amd.codegen.program import program_text
 from kunquant_amd.runner import KunRunner as kr
 from kunquant_amd.workloads import catalog
+from oracle import kun_oracle as ko
 from oracle.kun_oracle import OracleProgram
 from tests.helpers import assert_bit_exact
 
@@ -90,3 +91,19 @@ def _rank_rows(S, dt, seed):
 def test_rank_buckets(executor, module, S):
     dt = catalog.load(module)[1].dtype
     _check(executor, module, _rank_rows(S, dt, S), _rank_rows(S, dt, S + 1)[::-1].copy())
+
+
+@pytest.mark.parametrize("rank_inputs", [False, True])
+@pytest.mark.parametrize("S,T,n", [(1, 1, 1), (5, 9, 2), (127, 8, 3), (128, 7, 1), (129, 17, 17), (256, 64, 33), (1000, 5, 2)])
+def test_corr_tiles(executor, S, T, n, rank_inputs):
+    """Rows and tiles that do not fill up, more inputs than one launch takes,
+    signed zeros, a missing cell."""
+    rng = np.random.default_rng(S * 100 + T + n)
+    y = rng.standard_normal((T, S)).astype(np.float32)
+    y[0] = -0.0
+    xs = [rng.standard_normal((T, S)).astype(np.float32) for _ in range(n)]
+    xs[0][T // 2, S // 2] = np.nan
+    outs = [np.full(T, 7.0, np.float32) for _ in range(n)]
+    kr.corrWith(executor, xs, y, outs, "TS", rank_inputs=rank_inputs)
+    for x, o in zip(xs, outs):
+        assert_bit_exact(o, ko.corr_with(x, y, rank_inputs=rank_inputs), f"S={S} T={T} n={n}")

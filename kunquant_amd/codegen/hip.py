@@ -31,7 +31,7 @@ import numpy as np
 
 from ..Driver import BUF_INPUT, BUF_TEMP, ModuleIR, STAGE_GENERIC, STAGE_TS
 from ..Op import ConstantOp, ForeachBackWindow, Input, OpBase, Output, ReductionOp
-from .plan import PAR, SEQ, Component, StagePlan, plan_stage
+from .plan import PAR, SEQ, Component, StagePlan, plan_stage, rows_splittable
 from .program import literal, program_text
 from .wire import wire_table
 
@@ -106,7 +106,8 @@ _LAG_OPS = ("BackRef", "FastWindowedSum", "WindowedLinearRegression")
 _OP_COST = {"Div": 10, "DivConst": 10, "Sqrt": 8, "Log": 24, "Exp": 24, "IterValue": 2, "Select": 2,
             "ReduceAdd": 4, "ReduceMin": 4, "ReduceMax": 4, "ReduceArgMax": 7, "ReduceArgMin": 7,
             "ReduceRank": 6, "ReduceDecayLinear": 2, "FastWindowedSum": 16, "ExpMovingAvg": 8,
-            "WindowedLinearRegression": 30, "SkipListState": 60, "ForeachBackWindow": 2}
+            "WindowedLinearRegression": 30, "ForeachBackWindow": 2}
+SORTED_SLOT_COST = 6  # of a sorted window, per slot
 MAX_COMPS = 64
 # upper LDS bytes of the launch classes a level's components are split into
 # (16, 8, 4, 2 and 1 workgroups of 64 lanes per CU; the 80 KiB class is
@@ -418,7 +419,8 @@ class _Lowering:
             else:
                 L.append(f"const {T} {out} = ({T})st{src}.resi({w}, ({self.AT})({ins[1]}));")
         elif name == "SkipListState":
-            L.append(f"st{k}.step({ins[0]}, {ins[1]}, (int32_t)({time_idx}), {self.lane_expr(k)});")
+            L.append(f"st{k}.step({self.sorted_old(op, ins[0])}, {ins[1]}, (int32_t)({time_idx}), "
+                     f"{self.lane_expr(k)});")
             L.append(f"const {T} {out} = 0;")
         elif name in ("SkipListQuantile", "SkipListRank", "SkipListMin", "SkipListMax", "SkipListArgMin"):
             src = self.idx[op.inputs[0]]
@@ -440,6 +442,10 @@ class _Lowering:
             raise RuntimeError(f"HIP emitter: unsupported op {name}")
         L.extend(self.after_value(k))
         return L
+
+    def sorted_old(self, op, old: str) -> str:
+        """The value leaving a sorted window at this row."""
+        return old
 
     # None: the emitter has no in-run copy of window loops
     fast_win = None
@@ -816,8 +822,10 @@ class CompEmitter(_Lowering):
         # it sizes the rings.
         self.cost = self._cost()
         has_loop = any(isinstance(op, ForeachBackWindow) for op in self.ops)
+        # a sorted window is carried from row to row: its rows are not interleaved
+        has_sorted = any(op.__class__.__name__ == "SkipListState" for op in self.ops)
         self.interleave = 0
-        if kind == PAR and has_loop:
+        if kind == PAR and has_loop and not has_sorted:
             p = next((pp for c, pp in PAR_UNROLL_BY_COST if self.cost >= c), 8)
             p = min(max(p, INTERLEAVE_MIN), INTERLEAVE_MAX)
             p = max(1, min(p, PREFETCH_REGS // max(1, len(self.srcs) + len(self.lags))))
@@ -852,9 +860,9 @@ class CompEmitter(_Lowering):
             self.ring[self.idx[op]] = (slots, n_t)
             n_t += slots
         n_i = 0
-        # sorted windows of a sequential component live in registers while
-        # they fit SORTED_REGS values (with row indices where an argmin reads
-        # them), else in HBM scratch columns
+        # sorted windows live in registers while they fit SORTED_REGS values
+        # (with row indices where an argmin reads them), else in HBM scratch
+        # columns
         self.sorted_regs: Dict[int, bool] = {}
         regs = 0
         for op in self.ops:
@@ -863,7 +871,7 @@ class CompEmitter(_Lowering):
                 k = self.idx[op]
                 idx = any(o.__class__.__name__ == "SkipListArgMin" and o.inputs[0] is op for o in self.ops)
                 need = (w + 1) * (2 if idx else 1)
-                if kind == SEQ and regs + need <= SORTED_REGS:
+                if regs + need <= SORTED_REGS:
                     regs += need
                     self.sorted_regs[k] = idx
                     continue
@@ -881,7 +889,11 @@ class CompEmitter(_Lowering):
         # need deeper prefetch to cover HBM latency.
         self.depth = 1
         nload = max(1, sum(1 for op in self.srcs if self._src_row_used(op)) + len(self.lags))
-        if kind == PAR:
+        if has_sorted:
+            # one copy of the row: hundreds of instructions a window, which
+            # cover the next row's loads
+            p = 1
+        elif kind == PAR:
             p = next((pp for c, pp in PAR_UNROLL_BY_COST if self.cost >= c), 8)
         elif has_loop:
             p = SEQ_LOOP_UNROLL
@@ -905,13 +917,16 @@ class CompEmitter(_Lowering):
             if isinstance(op, (Input, ConstantOp)):
                 continue
             c = _OP_COST.get(op.__class__.__name__, 1)
+            if op.__class__.__name__ == "SkipListState":
+                c = SORTED_SLOT_COST * op.attrs["window"]
             loop = op.get_loop() if isinstance(op, ReductionOp) else op.get_parent()
             total += c * (loop.attrs["window"] if loop is not None else 1)
         return max(1, total)
 
     def _halo(self) -> int:
         """Rows of history a PAR chunk recomputes before its first stored row:
-        the longest chain of in-component window offsets."""
+        the longest chain of in-component window offsets. A sorted window
+        has to see its whole window, whoever computed the values."""
         need: Dict[OpBase, int] = {op: 0 for op in self.ops}
         for op in reversed(self.ops):
             if op not in self.computed:
@@ -925,12 +940,13 @@ class CompEmitter(_Lowering):
                     add = op.inputs[0].attrs["window"] - 1
                 elif name in _LAG_OPS and j == 0:
                     add = op.attrs["window"]
-                elif isinstance(op, ForeachBackWindow):
+                elif isinstance(op, ForeachBackWindow) or name == "SkipListState":
                     add = op.attrs["window"] - 1
                 else:
                     add = 0
                 need[inp] = max(need[inp], n + add)
-        return max((need[op] for op in self.computed), default=0)
+        return max((need[op] + (op.attrs["window"] - 1 if op.__class__.__name__ == "SkipListState" else 0)
+                    for op in self.computed), default=0)
 
     @property
     def lds_bytes(self) -> int:
@@ -1039,6 +1055,11 @@ class CompEmitter(_Lowering):
 
     def input_expr(self, op) -> str:
         raise AssertionError("row sources are loaded at the top of the row")
+
+    def sorted_old(self, op, old: str) -> str:
+        """Nothing leaves a chunk's sorted window that entered before the
+        chunk's first row."""
+        return f"kun::nan_before({old}, i - {op.attrs['window']} - rbeg)" if self.kind == PAR else old
 
     def output_lines(self, op, val: str) -> List[str]:
         if not self.emit_stores or op in self.shadow:
@@ -1301,13 +1322,13 @@ class LevelKernel:
     first) and maps a workgroup to (entry, chunk, 64-stock block)."""
 
     def __init__(self, module: ModuleIR, stage, plan: StagePlan, level, kname: str, lds_budget: int = None,
-                 comps=None):
+                 comps=None, kind: int = None):
         self.kname = kname
-        self.kind = level.kind
+        self.kind = kind = level.kind if kind is None else kind
         comps = level.comps if comps is None else comps
         if len(comps) > MAX_COMPS:
             raise RuntimeError(f"stage {stage.name}: {len(comps)} components in one kernel (limit {MAX_COMPS})")
-        self.comps = [CompEmitter(module, stage, plan, c, level.kind, lds_budget) for c in comps]
+        self.comps = [CompEmitter(module, stage, plan, c, kind, lds_budget) for c in comps]
         self.T = self.comps[0].T
         self.halo = max(c.halo for c in self.comps)
         self.lds_bytes = max(c.lds_bytes for c in self.comps)
@@ -1498,23 +1519,30 @@ def emit_module_parts(module: ModuleIR, nparts: int, lds_budget: int = None) -> 
             for level in plan.levels:
                 # one launch per LDS class, so that components with small
                 # rings are not held to the occupancy of the largest
-                classes: Dict[int, list] = {}
+                classes: Dict[Tuple[int, int], list] = {}
                 for c in level.comps:
-                    lds = CompEmitter(module, st, plan, c, level.kind, lds_budget).lds_bytes
-                    if level.kind == PAR:
+                    # components of a sequential level without a recurrence
+                    # over all rows run row-chunked, unless their windows
+                    # need scratch columns (one set per chunk would multiply
+                    # the run's device memory)
+                    kind = level.kind
+                    if rows_splittable(plan, c) and not CompEmitter(module, st, plan, c, PAR, lds_budget).spill_bytes:
+                        kind = PAR
+                    lds = CompEmitter(module, st, plan, c, kind, lds_budget).lds_bytes
+                    if kind == PAR:
                         cls = next(j for j, lim in enumerate(LDS_CLASSES) if lds <= lim)
                     else:
                         # sequential levels stay one launch (they are
                         # latency-bound) but for components past 40 KiB,
                         # which would hold every workgroup of it to two per CU
                         cls = 0 if lds <= 40 * 1024 else 1
-                    classes.setdefault(cls, []).append(c)
+                    classes.setdefault((kind, cls), []).append(c)
                 groups = []
-                for cls in sorted(classes):
-                    cl = classes[cls]
-                    groups.extend(cl[g:g + MAX_COMPS] for g in range(0, len(cl), MAX_COMPS))
-                for group in groups:
-                    lk = LevelKernel(module, st, plan, level, f"{kname}_k{len(kerns)}", lds_budget, group)
+                for kind, cls in sorted(classes):
+                    cl = classes[kind, cls]
+                    groups.extend((kind, cl[g:g + MAX_COMPS]) for g in range(0, len(cl), MAX_COMPS))
+                for kind, group in groups:
+                    lk = LevelKernel(module, st, plan, level, f"{kname}_k{len(kerns)}", lds_budget, group, kind)
                     if split:
                         kernel_srcs.append((lk.kname, lk.source()))
                     else:

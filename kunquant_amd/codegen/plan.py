@@ -5,7 +5,11 @@ The ops of a stage split into two classes:
     ExpMovingAvg, WindowedLinearRegression sums, SkipListState, and the
     Accumulator webs: the value at row t depends on every row since the run
     start through floating-point rounding, so each stock walks its rows in
-    order (the reference's semantics, Ops.hpp:300-375, 410-440);
+    order (the reference's semantics, Ops.hpp:300-375, 410-440). A sorted
+    window (SkipListState) is carried from row to row as well, but holds
+    nothing beyond its window: a component of a sequential level with no
+    other recurrence is emitted with its rows in chunks (rows_splittable),
+    each chunk filling its windows from empty over the rows before it;
   * window-pure ops -- elementwise ops, BackRef, window loops and their
     reductions: the value at row t is a fixed function of at most the last
     `w` rows of the op's inputs, so any range of rows can be computed
@@ -35,6 +39,44 @@ BOUND_OPS = {"WindowedLinearRegressionRSqaureImpl", "WindowedLinearRegressionSlo
              "WindowedLinearRegressionResiImpl", "SkipListQuantile", "SkipListRank", "SkipListMin",
              "SkipListMax", "SkipListArgMin"}
 ACC_OPS = {"Accumulator", "SetAccumulator"}
+
+
+_COPIES = ("Output", "WindowedTempOutput", "ReturnFirstValue")
+
+
+def _value(op: OpBase) -> OpBase:
+    """The op whose value `op` hands on unchanged."""
+    while op.__class__.__name__ in _COPIES:
+        op = op.inputs[0]
+    return op
+
+
+def is_window_sorted(op: OpBase) -> bool:
+    """True for a SkipListState whose leaving value is its entering value
+    `window` rows earlier (the only form the windowed ops build): its state at
+    row t is the sorted window of rows t - window + 1 .. t whatever came
+    before, so it can be rebuilt from any row on."""
+    old, cur = op.inputs[0], op.inputs[1]
+    return (old.__class__.__name__ == "BackRef" and old.attrs["window"] == op.attrs["window"]
+            and _value(old.inputs[0]) is _value(cur))
+
+
+def rows_splittable(plan: "StagePlan", comp: "Component") -> bool:
+    """True when a component of a sequential level holds nothing that depends
+    on every row since the run start: its rows can be computed in chunks like
+    those of a row-parallel level."""
+    if plan.fallback not in (None, "accumulator"):
+        return False
+    for op in comp.ops:
+        name = op.__class__.__name__
+        if name == "SkipListState":
+            if not is_window_sorted(op):
+                return False
+        elif name in REC_OPS or name in ACC_OPS or name.startswith("WindowedLinearRegression"):
+            return False
+        elif op.get_parent() is not None and op.get_parent().get_parent() is not None:
+            return False
+    return True
 
 
 def is_source(op: OpBase) -> bool:

@@ -341,61 +341,58 @@ template <typename T, int W> struct SortedWin {
     }
 };
 
-// The same sorted window held in registers by a lane that walks every row
-// of the run (sequential batch kernels): every access uses a compile-time
-// slot, so insertion and removal are W + 1 selects instead of a chain of
-// dependent memory round trips. IDX keeps the row indices (SkipListArgMin).
-// Ordering is that of SortedWin: a new value goes after equal ones, a
-// removal takes the first equal one.
+// The same sorted window held in registers (batch kernels): W slots that are
+// always all in use, a missing value being a slot of +inf at its place in the
+// order of arrival. One row takes the oldest arrival out and puts the newest
+// in, in one pass of compile-time slots. Equal values, the empty slots among
+// them, stand in order of arrival, so the first of them is the one to leave
+// and a new one goes after the last (SortedWin's order); quantities of the
+// window are read only while all W values are there (n == W), when no empty
+// slot is left. IDX keeps the row indices (SkipListArgMin).
+//
+// 2 compares and 3 selects a slot and row; searching, shifting and storing
+// in separate passes with a count of used slots took about four times that.
 template <typename T, int W, bool IDX> struct SortedWinR {
-    T v[W + 1];
-    int32_t ix[IDX ? W + 1 : 1];
+    T v[W];
+    int32_t ix[IDX ? W : 1];
     int n = 0, last = 0;
     __device__ __forceinline__ SortedWinR() {
 #pragma unroll
-        for (int k = 0; k <= W; k++) v[k] = T(0);
+        for (int k = 0; k < W; k++) v[k] = inf<T>();
 #pragma unroll
-        for (int k = 0; k < (IDX ? W + 1 : 1); k++) ix[k] = 0;
+        for (int k = 0; k < (IDX ? W : 1); k++) ix[k] = 0;
     }
     __device__ __forceinline__ void step(T old, T cur, int32_t index, long) {
-        if (old == old) {
-            int p = 0;
+        n += (cur == cur ? 1 : 0) - (old == old ? 1 : 0);
+        const T o = old == old ? old : inf<T>();
+        const T c = cur == cur ? cur : inf<T>();
+        int pos = 0;
+        // slot k of the window without the leaving value is d, the slot
+        // before it p; `le` and `ple` tell whether they go before c
+        T p = c;
+        int32_t px = index;
+        bool ple = true;
 #pragma unroll
-            for (int k = 0; k <= W; k++) p += (k < n && v[k] < old) ? 1 : 0;
-            bool found = false;
-#pragma unroll
-            for (int k = 0; k <= W; k++) found = found || (k == p && k < n && v[k] == old);
-            if (found) {
-#pragma unroll
-                for (int k = 0; k < W; k++) {
-                    v[k] = k >= p ? v[k + 1] : v[k];
-                    if (IDX) ix[k] = k >= p ? ix[k + 1] : ix[k];
-                }
-                n--;
+        for (int k = 0; k < W; k++) {
+            const bool keep = k == W - 1 ? false : v[k] < o;
+            const T d = keep ? v[k] : (k < W - 1 ? v[k + 1] : inf<T>());
+            const bool le = k < W - 1 && d <= c;
+            pos += le ? 1 : 0;
+            if (IDX) {
+                const int32_t dx = keep ? ix[k] : (k < W - 1 ? ix[k + 1] : 0);
+                ix[k] = le ? dx : (ple ? index : px);
+                px = dx;
             }
+            v[k] = le ? d : (ple ? c : p);
+            p = d;
+            ple = le;
         }
-        if (cur == cur) {
-            int p = 0;
-#pragma unroll
-            for (int k = 0; k <= W; k++) p += (k < n && v[k] <= cur) ? 1 : 0;
-#pragma unroll
-            for (int k = W; k > 0; k--) {
-                v[k] = k > p ? v[k - 1] : v[k];
-                if (IDX) ix[k] = k > p ? ix[k - 1] : ix[k];
-            }
-#pragma unroll
-            for (int k = 0; k <= W; k++) {
-                v[k] = k == p ? cur : v[k];
-                if (IDX) ix[k] = k == p ? index : ix[k];
-            }
-            n++;
-            last = p;
-        }
+        last = pos;
     }
     __device__ __forceinline__ T at(int i) const {
         T r = T(0);
 #pragma unroll
-        for (int k = 0; k <= W; k++) r = k == i ? v[k] : r;
+        for (int k = 0; k < W; k++) r = k == i ? v[k] : r;
         return r;
     }
     __device__ __forceinline__ T quantile(T q, long) const {

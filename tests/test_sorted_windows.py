@@ -1,0 +1,93 @@
+"""Sorted windows (quantile, and the skip-list forms of rank, extremes and
+position) in row chunks: the generated kernels run on the CPU against the
+oracle bit for bit, for chunks around the window's length, with missing
+values, ties, zeros of both signs and infinities."""
+import numpy as np
+import pytest
+
+from emu.emu import EmuModule
+from kunquant_amd.codegen.hip import rows_splittable, stage_plan
+from kunquant_amd.codegen.plan import is_window_sorted
+from kunquant_amd.codegen.program import program_text
+from kunquant_amd.Driver import compileit
+from kunquant_amd.Op import Builder, Input, Output
+from kunquant_amd.Stage import Function
+from kunquant_amd.ops import BackRef, ExpMovingAvg, SkipListQuantile, SkipListState, WindowedQuantile
+from kunquant_amd.ops.MiscOp import SkipListArgMin, SkipListMax, SkipListMin, SkipListRank
+from oracle.kun_oracle import OracleProgram
+from tests.helpers import assert_bit_exact
+
+
+def _graph(w):
+    b = Builder()
+    with b:
+        a = Input("a")
+        Output(WindowedQuantile(a, w, 0.3), "q")
+        Output(WindowedQuantile(a * 2 - BackRef(a, 2), w, 0.8), "q_computed")
+        st = SkipListState(BackRef(a, w), a, w)
+        Output(SkipListRank(st, a), "rank")
+        Output(SkipListMin(st), "min")
+        Output(SkipListMax(st), "max")
+        Output(SkipListArgMin([st], []), "argmin")
+    return Function(b.ops)
+
+
+def _rows(T, S, dt):
+    rng = np.random.default_rng(T + S)
+    a = rng.standard_normal((T, S))
+    a[:, 1] = np.round(a[:, 1] * 2)                                     # ties
+    a[:, 2] = rng.choice([0.0, -0.0, 1.0], T)
+    a[:, 3] = rng.choice([np.inf, -np.inf, 0.5, np.nan], T)
+    a[:, 4] = np.where(rng.random(T) < 0.1, np.nan, a[:, 4])
+    a[:, 5] = np.nan
+    a[:, 6] = np.inf
+    a[:, 7] = np.arange(T)
+    return np.ascontiguousarray(a.astype(dt))
+
+
+@pytest.mark.parametrize("dtype", ["float", "double"])
+@pytest.mark.parametrize("w", [1, 2, 7, 150])
+def test_row_chunks_equal_the_oracle(dtype, w):
+    """150 rows: the values and row indices of the one state exceed the
+    registers, sit in scratch columns and keep walking every row."""
+    m = compileit(_graph(w), f"sorted{w}_{dtype}", input_layout="TS", output_layout="TS", dtype=dtype,
+                  options={"no_fast_stat": "no_warn"})
+    S, T, start = 9, 2 * w + 40, 3
+    L = T - start
+    a = _rows(T, S, np.float32 if dtype == "float" else np.float64)
+    exp = OracleProgram(program_text(m)).run({"a": a}, S, T, start, L, nthreads=2, temps=True)
+    emu = EmuModule(m)
+    for st in m.stages:
+        for chunk in {0, 1, max(1, w - 1), w, w + 1, 16}:
+            got = {"a": a, **exp}
+            for b in st.out_bufs:
+                got[b.name] = np.full_like(exp[b.name], 12345.0)
+            emu.run_stage(st.idx, got, S, T, start, L, chunk)
+            for b in st.out_bufs:
+                assert_bit_exact(got[b.name], exp[b.name], f"{b.name} chunk {chunk}")
+
+
+def test_only_pure_windows_are_split():
+    """A state fed something else than its own value a window ago, and one
+    beside a recurrence over all rows, keep walking every row."""
+    b = Builder()
+    with b:
+        a = Input("a")
+        good = SkipListState(BackRef(a, 9), a, 9)
+        other = SkipListState(BackRef(a, 8), a, 9)
+        Output(SkipListQuantile(good, 0.5), "good")
+        Output(SkipListQuantile(other, 0.5), "other")
+        Output(ExpMovingAvg(a, 5), "ema")
+    m = compileit(Function(b.ops), "t", input_layout="TS", output_layout="TS", dtype="double",
+                  options={"no_fast_stat": "no_warn"})
+    (st,) = m.stages
+    plan = stage_plan(m, st)
+    split = {}
+    for level in plan.levels:
+        for c in level.comps:
+            for op in c.ops:
+                if isinstance(op, Output):
+                    split[op.attrs["name"]] = rows_splittable(plan, c)
+                if op.__class__.__name__ == "SkipListState":
+                    assert is_window_sorted(op) == (op.inputs[0].attrs["window"] == 9)
+    assert split == {"good": True, "other": False, "ema": False}

@@ -90,10 +90,11 @@ PAR_UNROLL_BY_COST = ((1024, 1), (256, 2), (64, 4))
 # the scheduler lifts every row's NaN select of its lag value to the top of
 # the 16-row iteration, where it waits for loads issued a row earlier
 ROW_BARRIER = 0x9C
-# row-chunked components with window loops: rows per interleaved group
-# (2: at two waves per SIMD, wider groups cost more in registers than they
-# gain in overlapped chains; measured against 1, 3 and 4)
-INTERLEAVE_MIN, INTERLEAVE_MAX = 2, 2
+# row-chunked components with window loops: rows per interleaved group. Rows
+# share the group's window reads, so that four rows cost few more registers
+# than two: 2 / 3 / 4 rows ran the 100-factor fp32 graph in 26.6 / 25.9 /
+# 25.4 ms (row-chunked kernels alone 18.8 / 17.6 / 17.1)
+INTERLEAVE_MIN, INTERLEAVE_MAX = 4, 4
 
 _BIN = {"Add": "+", "Sub": "-", "Mul": "*", "Div": "/"}
 _CMP = {"GreaterThan": ">", "GreaterEqual": ">=", "LessThan": "<", "LessEqual": "<=", "Equals": "=="}
@@ -195,14 +196,20 @@ _DEF = re.compile(r"\bconst\s+\w+\s+(\w+)\s*=")
 _ITER = re.compile(r"\biter\b")
 
 
-def loop_code(w: int, body: List[str], unroll: int) -> List[str]:
+_ELEM = re.compile(r"\bXE\((\d+),(\d+)\)")
+
+
+def loop_code(w: int, body: List[str], unroll: int, loads=None) -> List[str]:
     """A window loop over iter = w-1 .. 0 (oldest value first), unrolled by
     hand in groups of `unroll` iterations (0: the whole window): the group's
-    window reads -- statements that depend on nothing but `iter` -- are
-    issued first, then the iterations run in order. Every statement of the
-    loop body keeps its order relative to the others of its iteration, so
-    the arithmetic is that of the plain loop; only the loads move earlier,
-    so that their latency overlaps the dependent chains."""
+    window reads come first -- statements that depend on nothing but `iter`,
+    and the elements that `loads(n, first)` reads for n iterations from
+    iter = `first` on (see CompEmitter.elem_loads) -- then the iterations run
+    in order. Every statement of the loop body keeps its order relative to
+    the others of its iteration, so the arithmetic is that of the plain loop;
+    only the loads move earlier, so that their latency overlaps the dependent
+    chains. XE(k,q) in a statement is the value of source k that row q of an
+    interleaved group reads in that iteration: element q + u of the group."""
     U = w if unroll <= 0 else min(unroll, w)
     defined = set()
     for x in body:
@@ -215,6 +222,7 @@ def loop_code(w: int, body: List[str], unroll: int) -> List[str]:
         out = []
         for x in body:
             x = _ITER.sub(f"(it0 - {u})", x)
+            x = _ELEM.sub(lambda m: f"x{m.group(1)}_{int(m.group(2)) + u}", x)
             for n in defined:
                 x = re.sub(rf"\b{n}\b", f"{n}u{u}", x)
             out.append(x)
@@ -222,14 +230,15 @@ def loop_code(w: int, body: List[str], unroll: int) -> List[str]:
 
     def group(n: int) -> List[str]:
         copies = [copy(u) for u in range(n)]
-        G = []
+        G = list(loads(n, "it0")) if loads else []
         for c in copies:
             G.extend(c[i] for i in hoist)
         for c in copies:
             G.extend(c[i] for i in range(len(c)) if i not in hoist)
         return G
 
-    L = ["{", "int it0 = " + str(w - 1) + ";", f"for (; it0 >= {U - 1}; it0 -= {U}) {{"]
+    L = ["{", "int it0 = " + str(w - 1) + ";"] + (["#pragma nounroll"] if loads else [])
+    L.append(f"for (; it0 >= {U - 1}; it0 -= {U}) {{")
     L.extend(group(U))
     L.append("}")
     if w % U:
@@ -237,29 +246,33 @@ def loop_code(w: int, body: List[str], unroll: int) -> List[str]:
         # groups measured no faster in batch kernels and slower in stream
         # tick kernels, whose window reads come from HBM)
         L.append("for (int iter = it0; iter >= 0; --iter) {")
-        L.extend(body)
+        if loads:
+            L.extend(loads(1, "iter"))
+        L.extend(_ELEM.sub(lambda m: f"x{m.group(1)}_{m.group(2)}", x) for x in body)
         L.append("}")
     L.append("}")
     return L
 
 
-def window_loop(w: int, body: List[str], fast: Optional[List[str]], unroll: int, row: str = "i") -> List[str]:
-    """loop_code of a window loop; with an in-run body, that copy runs when
-    every row the loop reads lies in the run (`row` >= w - 1, `row` being
-    the lowest row of the loop) and the buffers allow kun::wld."""
+def window_loop(w: int, body: List[str], unroll: int, loads=None, fast=None, row: str = "i") -> List[str]:
+    """loop_code of a window loop; with in-run loads (`fast`), the copy using
+    them runs when every row the loop reads lies in the run (`row` >= w - 1,
+    `row` being the lowest row of the loop) and the buffers allow kun::wld."""
     if fast is None:
-        return loop_code(w, body, unroll)
-    return ([f"if (wok && {row} >= {w - 1}) {{"] + loop_code(w, fast, unroll) + ["} else {"]
-            + loop_code(w, body, unroll) + ["}"])
+        return loop_code(w, body, unroll, loads)
+    return ([f"if (wok && {row} >= {w - 1}) {{"] + loop_code(w, body, unroll, fast) + ["} else {"]
+            + loop_code(w, body, unroll, loads) + ["}"])
 
 
-def _flatten(segs, unroll: int) -> List[str]:
+def _flatten(segs, unroll: int, loads_of=lambda srcs: (None, None)) -> List[str]:
     L = []
     for sg in segs:
         if sg[0] == "lines":
             L.extend(sg[1])
         else:
-            L.extend(sg[1] + window_loop(sg[2], sg[3], sg[5], unroll) + sg[4])
+            loads, fast = loads_of(sg[5])
+            L.extend(sg[1] + window_loop(sg[2], [x.replace("XE(@", "XE(").replace("@)", ",0)") for x in sg[3]], unroll,
+                                         loads, fast) + sg[4])
     return L
 
 
@@ -385,7 +398,7 @@ class _Lowering:
         elif name == "Select":
             L.append(f"const {T} {out} = kun::sel({ins[0]}, {ins[1]}, {ins[2]});")
         elif name == "IterValue":
-            L.append(f"const {T} {out} = {self.win(op.inputs[1], 'iter')};")
+            L.append(f"const {T} {out} = {self.iter_read(op.inputs[1])};")
         elif name == "WindowLoopIndex":
             w = op.inputs[0].attrs["window"]
             L.append(f"const {T} {out} = ({T})({w} - 1 - iter);")
@@ -447,15 +460,14 @@ class _Lowering:
         """The value leaving a sorted window at this row."""
         return old
 
-    # None: the emitter has no in-run copy of window loops
-    fast_win = None
+    def iter_read(self, src) -> str:
+        """The value a window loop reads in iteration `iter`."""
+        return self.win(src, "iter")
 
     def loop_parts(self, loop):
-        """(declarations, window, loop body, finalisation, in-run body) of a
-        window loop (see loop_code). The in-run body, when the emitter has
-        one and it differs, reads row sources without the clamp and NaN
-        select that rows before the run start need; it is correct for rows
-        i >= window - 1 and reads the same values there."""
+        """(declarations, window, loop body, finalisation, sources) of a
+        window loop (see loop_code); the sources are those that the body
+        reads as elements XE."""
         T = self.T
         w = loop.attrs["window"]
         body = [op for op in self.ops if op.get_parent() is loop]
@@ -503,16 +515,7 @@ class _Lowering:
                 raise RuntimeError(f"HIP emitter: unsupported reduction {name}")
         pre = L
         body_lines = self._loop_body(body, reds)
-        fast = None
-        if self.fast_win is False:
-            # the copy for rows whose window lies inside the run (row >= w - 1)
-            self.fast_win = True
-            try:
-                fast = self._loop_body(body, reds)
-            finally:
-                self.fast_win = False
-            if fast == body_lines:
-                fast = None
+        seen = {int(k) for x in body_lines for k in re.findall(r"\bXE\(@(\d+)@\)", x)}
         L = []
         for r in reds:
             k = self.idx[r]
@@ -526,7 +529,7 @@ class _Lowering:
             elif name == "ReduceRank":
                 L.append(f"v{k} = r{k}_lt + (r{k}_eq + {T}(1.0)) / {T}(2.0);")
             L.extend(self.after_value(k))
-        return pre, w, body_lines, L, fast
+        return pre, w, body_lines, L, sorted(seen)
 
     def _loop_body(self, body, reds) -> List[str]:
         T = self.T
@@ -575,7 +578,11 @@ class _Lowering:
         return segs
 
     def step_lines(self, skip=()) -> List[str]:
-        return _flatten(self.step_segments(skip), self.loop_unroll)
+        return _flatten(self.step_segments(skip), self.loop_unroll, self.loads_of)
+
+    def loads_of(self, srcs):
+        """(loads, in-run loads) of a loop's element sources for window_loop."""
+        return None, None
 
     def buffer_ptrs(self, args: str = "A") -> List[str]:
         T = self.T
@@ -1013,22 +1020,64 @@ class CompEmitter(_Lowering):
         """The load of lag_load without its NaN select (row clamped at 0)."""
         return self.src_load(op, f"(({row}) < 0 ? 0 : ({row}))")
 
-    # set while lowering the copy of a window loop that runs when every row
-    # the loop reads lies inside the run (see loop_parts)
-    fast_win = False
+    def iter_read(self, src) -> str:
+        return f"XE(@{self.idx[src]}@)"
 
-    def in_run_load(self, op, row: str) -> str:
-        """Row `row` (>= 0) of a row source: no clamp, no NaN select. [rows][S]
-        buffers load through kun::wld (row offset in a scalar register)."""
-        k = self.idx[op]
-        e = self.esz
+    def loads_of(self, srcs, P: int = 1):
+        """Element loads of a window loop over P interleaved rows (rows iq0 ..
+        of a group, or row i alone), and the in-run ones where a source is
+        read straight from HBM."""
+        ops = [self.st.func.ops[k] for k in srcs]
+        sfx = "q0" if P > 1 else ""
+        loads = lambda n, it: [x for op in ops for x in self.elem_loads(op, n + P - 1, it, sfx, False)]
+        if not any(self.idx[op] not in self.ring for op in ops):
+            return loads, None
+        return loads, lambda n, it: [x for op in ops for x in self.elem_loads(op, n + P - 1, it, sfx, True)]
+
+    def elem_loads(self, op, n: int, it: str, sfx: str, in_run: bool) -> List[str]:
+        """x<k>_0 .. x<k>_<n-1>: rows i - `it` .. of source k, i being the
+        first row of the loop: what an unrolled group of iterations reads, and
+        in an interleaved group every row's reads, each once.
+
+        A ring's rows are consecutive slots but where it ends: unless the
+        elements cross its end they have one address and constant offsets (two
+        elements to an LDS instruction), instead of a wrapped slot, its
+        address and a read for every row and iteration: about 7 instructions
+        an element instead of 13, most of the others scalar, which a SIMD
+        with two or three wavefronts pays for in full. A 60-row deviation
+        over 8192 x 1024 floats: 211 -> 175 us with two rows a group; the
+        100-factor graph's row-chunked kernels 20.7 -> 18.8 ms."""
+        T, k = self.T, self.idx[op]
+        names = [f"x{k}_{e}" for e in range(n)]
+        if k in self.ring:
+            slots, base = self.ring[k]
+            in_lds = base < self.lds_t
+            at = lambda slot: self.tmem(f"{base} + {slot}", base)
+            L = [f"int g{k} = rp{k}{sfx} - ({it}); g{k} = g{k} < 0 ? g{k} + {slots} : g{k};"]
+            wrapped = [f"{x} = {at(f'(g{k} + {e} < {slots} ? g{k} + {e} : g{k} - {slots - e})')};"
+                       for e, x in enumerate(names)]
+            if slots < n + 4:  # (almost) every group crosses the end
+                return L + [f"const {T} " + x for x in wrapped]
+            step = "64" if in_lds else "cst"
+            return (L + [f"{T} {', '.join(names)};", f"if (g{k} < {slots - n + 1}) {{",
+                         f"const {T} *r{k} = &{at(f'g{k}')};"]
+                    + [f"{x} = r{k}[{e} * {step}];" for e, x in enumerate(names)]
+                    # (keeps the two branches' loads from being merged into
+                    # one of selected addresses)
+                    + ['asm volatile("" ::: "memory");', "} else {"] + wrapped + ["}"])
+        if not in_run:
+            return [f"const {T} {x} = {self.lag_load(op, f'i{sfx} - ({it}) + {e}')};" for e, x in enumerate(names)]
         if isinstance(op, Input):
             b = self.m.buffer(op.attrs["name"])
             if self.buf_layout(op) != "1":
-                return self.src_load(op, row)
-            r = f"A.start + ({row})" if b.kind == BUF_INPUT else f"({row})"
-            return f"kun::wld(b{b.idx}, so, ({r}) * A.S * {e})"
-        return f"kun::wld(m{k}, so, ({row}) * A.S * {e})"
+                return [f"const {T} {x} = {self.src_load(op, f'i{sfx} - ({it}) + {e}')};" for e, x in enumerate(names)]
+            ptr, first = f"b{b.idx}", (f"A.start + i{sfx}" if b.kind == BUF_INPUT else f"i{sfx}")
+        else:
+            ptr, first = f"m{k}", f"i{sfx}"
+        # rows known to lie in the run: no clamp, no NaN select, the row
+        # offset in a scalar register (kun::wld)
+        return [f"const long ro{k} = ({first} - ({it})) * A.S * {self.esz};"] + [
+            f"const {T} {x} = kun::wld({ptr}, so, ro{k} + {e} * A.S * {self.esz});" for e, x in enumerate(names)]
 
     # ring reads of earlier rows hoisted to the top of the row being
     # emitted (see row_segments): None when not collecting
@@ -1047,11 +1096,7 @@ class CompEmitter(_Lowering):
             # single-offset read of a row source: its prefetched lag load (a
             # ring kept for the source's window loops may be shorter)
             return f"lg{k}_{off}"
-        if k in self.src_ring:
-            return self.ring_read(k, off)
-        if self.fast_win:
-            return self.in_run_load(src, f"i - ({off})")
-        return self.lag_load(src, f"i - ({off})")
+        raise AssertionError("window loops read their sources as elements")
 
     def input_expr(self, op) -> str:
         raise AssertionError("row sources are loaded at the top of the row")
@@ -1124,7 +1169,7 @@ class CompEmitter(_Lowering):
         """Statements of one row `i`. With the row body unrolled P > 1 times,
         prefetch slot q holds this row and is refilled P rows ahead; with
         P == 1 the slots form a shift register `depth` rows deep."""
-        return _flatten(self.row_segments(q, P), self.loop_unroll)
+        return _flatten(self.row_segments(q, P), self.loop_unroll, self.loads_of)
 
     def row_segments(self, q: int, P: int, grouped: bool = False) -> list:
         """row_lines as segments (see step_segments). Single-offset ring
@@ -1193,12 +1238,11 @@ class CompEmitter(_Lowering):
                 continue
             for q in range(P):
                 L.extend(_rename_row(segs[q][j][1], q, keep))
-            body, fast = [], []
+            body = []
             for q in range(P):
-                body.extend(_rename_row(segs[q][j][3], q, keep))
-                if sg[5] is not None:
-                    fast.extend(_rename_row(segs[q][j][5], q, keep))
-            L.extend(window_loop(sg[2], body, fast if sg[5] is not None else None, self.loop_unroll, "iq0"))
+                body.extend(x.replace("XE(@", "XE(").replace("@)", f",{q})") for x in _rename_row(segs[q][j][3], q, keep))
+            loads, fast = self.loads_of(sg[5], P)
+            L.extend(window_loop(sg[2], body, self.loop_unroll, loads, fast, "iq0"))
             for q in range(P):
                 L.extend(_rename_row(segs[q][j][4], q, keep))
         return L

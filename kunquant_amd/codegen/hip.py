@@ -1001,9 +1001,13 @@ class CompEmitter(_Lowering):
             b = self.m.buffer(op.attrs["name"])
             lay = self.buf_layout(op)
             if b.kind == BUF_INPUT:
+                if lay == "1":
+                    return f"kun::row_ld(b{b.idx} + sb, start + ({row}), S32, lo)"
                 return f"b{b.idx}[kun::at<{lay}>(A.start + ({row}), s, A.S, A.T, A.blk)]"
+            if lay == "1":
+                return f"kun::row_ld(b{b.idx} + sb, {row}, S32, lo)"
             return f"b{b.idx}[kun::at<{lay}>(({row}), s, A.S, A.L, A.blk)]"
-        return f"m{k}[(size_t)({row}) * A.S + s]"
+        return f"kun::row_ld(m{k} + sb, {row}, S32, lo)"
 
     def mat_buf(self, op) -> int:
         """Entry of kun::StageArgs::bufs holding materialised value `op`
@@ -1071,13 +1075,13 @@ class CompEmitter(_Lowering):
             b = self.m.buffer(op.attrs["name"])
             if self.buf_layout(op) != "1":
                 return [f"const {T} {x} = {self.src_load(op, f'i{sfx} - ({it}) + {e}')};" for e, x in enumerate(names)]
-            ptr, first = f"b{b.idx}", (f"A.start + i{sfx}" if b.kind == BUF_INPUT else f"i{sfx}")
+            ptr, first = f"b{b.idx}", (f"start + i{sfx}" if b.kind == BUF_INPUT else f"i{sfx}")
         else:
             ptr, first = f"m{k}", f"i{sfx}"
         # rows known to lie in the run: no clamp, no NaN select, the row
         # offset in a scalar register (kun::wld)
-        return [f"const long ro{k} = ({first} - ({it})) * A.S * {self.esz};"] + [
-            f"const {T} {x} = kun::wld({ptr}, so, ro{k} + {e} * A.S * {self.esz});" for e, x in enumerate(names)]
+        return [f"const unsigned ro{k} = (unsigned)({first} - ({it})) * rsz;"] + [
+            f"const {T} {x} = kun::wld({ptr}, so, ro{k} + {e} * rsz);" for e, x in enumerate(names)]
 
     # ring reads of earlier rows hoisted to the top of the row being
     # emitted (see row_segments): None when not collecting
@@ -1110,12 +1114,14 @@ class CompEmitter(_Lowering):
         if not self.emit_stores or op in self.shadow:
             return []
         b = self.m.buffer(op.attrs["name"])
+        if self.buf_layout(op) == "1":
+            return [f"kun::row_st(b{b.idx} + sb, i, S32, lo, {val});"]
         return [f"b{b.idx}[kun::at<{self.buf_layout(op)}>(i, s, A.S, A.L, A.blk)] = {val};"]
 
     def after_value(self, k: int) -> List[str]:
         L = self.ring_push(k)
         if self.emit_stores and self.st.func.ops[k] in self.plan.mat:
-            L.append(f"w{k}[(size_t)i * A.S + s] = v{k};")
+            L.append(f"kun::row_st(w{k} + sb, i, S32, lo, v{k});")
         return L
 
     # -- code -------------------------------------------------------------
@@ -1230,7 +1236,7 @@ class CompEmitter(_Lowering):
         the earlier rows' window reads."""
         keep = {self.idx[op] for op in self.single}
         segs = [self.row_segments(q, P, grouped=True) for q in range(P)]
-        L = [f"const long iq{q} = i0 + {q};" for q in range(P)]
+        L = [f"const int iq{q} = i0 + {q};" for q in range(P)]
         for j, sg in enumerate(segs[0]):
             if sg[0] == "lines":
                 for q in range(P):
@@ -1253,12 +1259,18 @@ class CompEmitter(_Lowering):
         T = self.T
         L = []
         if self.kind == PAR:
-            L.append("const long c0 = (long)chunk_id * A.zchunk[e];")
-            L.append("const long c1 = c0 + A.zchunk[e] < A.L ? c0 + A.zchunk[e] : A.L;")
-            L.append(f"const long rbeg = c0 - {self.halo} > 0 ? c0 - {self.halo} : 0;")
+            L.append("const int c0 = chunk_id * A.zchunk[e], nrow = (int)A.L;")
+            L.append("const int c1 = c0 + A.zchunk[e] < nrow ? c0 + A.zchunk[e] : nrow;")
+            L.append(f"const int rbeg = c0 - {self.halo} > 0 ? c0 - {self.halo} : 0;")
         else:
-            L.append("const long c0 = 0, c1 = A.L, rbeg = 0;")
+            L.append("const int c0 = 0, c1 = (int)A.L, rbeg = 0;")
             L.append("(void)c0;")
+        # rows and stocks in 32-bit scalars: 64-bit compares have no scalar
+        # form, and the address of a row is then two scalar products, a shift
+        # and an add, the lane's part a register that never changes (a rolling
+        # sum's row: 54 -> 37 instructions)
+        L.append("const int start = (int)A.start; (void)start;")
+        L.append(f"const unsigned S32 = (unsigned)A.S, rsz = S32 * {self.esz}u, lo = (unsigned)lane * {self.esz}u; (void)lo; (void)rsz;")
         # window loops whose rows all lie in the run take their in-run copy
         # (kun::wld) when every byte offset of the [rows][S] buffers fits
         # in 31 bits
@@ -1288,7 +1300,7 @@ class CompEmitter(_Lowering):
             # the LDS stores so they overlap
             PF = 8
             mo = max(self.src_ring.values())
-            L.append(f"for (long rb = rbeg - {mo} > 0 ? rbeg - {mo} : 0; rb < rbeg; rb += {PF}) {{")
+            L.append(f"for (int rb = rbeg - {mo} > 0 ? rbeg - {mo} : 0; rb < rbeg; rb += {PF}) {{")
             for k, off in sorted(self.src_ring.items()):
                 op = self.st.func.ops[k]
                 for q in range(PF):
@@ -1310,6 +1322,16 @@ class CompEmitter(_Lowering):
                     L.append(f"{T} pf{self.idx[op]}_{q} = {self.src_load(op, first)};")
             for (k, off) in self.lags:
                 L.append(f"{T} pl{k}_{off}_{q} = {self.lag_raw(self.st.func.ops[k], f'{first} - {off}')};")
+        if self.kind == SEQ and P > 1:
+            # The first loads land before the loop starts, so that every wait
+            # in it counts from the loop's own loads (vmcnt only, 0xF70). Else
+            # the wait at a slot's use is the smaller of what the loop and the
+            # loads before it (back to back, no stores between) allow: about
+            # the last third of the prefetch was waited for at the top of
+            # every group of rows. With the scalar row addresses, the
+            # sequential kernels of the 100-factor graph (8192 x 1024 floats),
+            # alone: 10.0 -> 7.0 ms.
+            L.append("__builtin_amdgcn_s_waitcnt(0xF70);")
         if self.kind == PAR:
             # halo rows rebuild history and store nothing; stored rows follow
             # in a phase of their own so neither phase branches on the row
@@ -1327,15 +1349,15 @@ class CompEmitter(_Lowering):
         groups, a guarded tail."""
         L = []
         if P == 1:
-            L.append(f"for (long i = {lo}; i < {hi}; ++i) {{")
+            L.append(f"for (int i = {lo}; i < {hi}; ++i) {{")
             L.extend("  " + x for x in self.row_lines(0, 1))
             L.append("}")
             return L
         L.append("{")
-        L.append(f"  long i0 = {lo} - {lo} % {P};")
+        L.append(f"  int i0 = {lo} - {lo} % {P};")
         if lo != "0":
             for q in range(P):
-                L.append(f"  {{ const long i = i0 + {q};")
+                L.append(f"  {{ const int i = i0 + {q};")
                 L.append(f"  if (i >= {lo} && i < {hi}) {{")
                 L.extend("    " + x for x in self.row_lines(q, P))
                 L.append("  } }")
@@ -1345,14 +1367,14 @@ class CompEmitter(_Lowering):
             L.extend("    " + x for x in self.group_lines(P))
         else:
             for q in range(P):
-                L.append(f"    {{ const long i = i0 + {q};")
+                L.append(f"    {{ const int i = i0 + {q};")
                 L.extend("      " + x for x in self.row_lines(q, P))
                 if ROW_BARRIER is not None:
                     L.append(f"      __builtin_amdgcn_sched_barrier({ROW_BARRIER});")
                 L.append("    }")
         L.append("  }")
         for q in range(P - 1):
-            L.append(f"  if (i0 + {q} < {hi}) {{ const long i = i0 + {q};")
+            L.append(f"  if (i0 + {q} < {hi}) {{ const int i = i0 + {q};")
             L.extend("    " + x for x in self.row_lines(q, P))
             L.append("  }")
         L.append("}")
@@ -1414,7 +1436,8 @@ class LevelKernel:
              "  const int nsb = (int)((A.S + 63) >> 6);",
              "  const int local = wg - A.zfirst[e];",
              "  const int chunk_id = local / nsb;",
-             f"  const long s = (long)(local - chunk_id * nsb) * {TS_BLOCK} + lane;"]
+             f"  const size_t sb = (size_t)(local - chunk_id * nsb) * {TS_BLOCK};",
+             "  const long s = (long)sb + lane;"]
         lds_t = max(c.lds_t for c in self.comps)
         if lds_t:
             L.append(f"  __shared__ {T} lds[{lds_t * TS_BLOCK}];")

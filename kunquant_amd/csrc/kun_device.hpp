@@ -439,6 +439,16 @@ template <typename T> __device__ __forceinline__ T wld(const T *base, unsigned s
     }
 }
 
+// Cell of the wavefront's lane in row `row` of a [rows][S] buffer: `base` is
+// the wavefront's first stock of row 0 and `lo` the lane's byte offset, so
+// that the address is a scalar one and a register that never changes.
+template <typename T> __device__ __forceinline__ T row_ld(const T *base, unsigned row, unsigned S, unsigned lo) {
+    return *(const T *)((const char *)(base + (size_t)row * S) + lo);
+}
+template <typename T> __device__ __forceinline__ void row_st(T *base, unsigned row, unsigned S, unsigned lo, T v) {
+    *(T *)((char *)(base + (size_t)row * S) + lo) = v;
+}
+
 // element (row, stock) of a buffer in TS [rows][S] or STs [S/b][rows][b]
 template <int LAYOUT> __device__ __forceinline__ size_t at(long row, long s, long S, long rows, int blk) {
     if (LAYOUT == 1) return (size_t)row * S + s;

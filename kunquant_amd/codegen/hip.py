@@ -482,17 +482,17 @@ class _Lowering:
             elif name == "ReduceMul":
                 L.append(f"{T} r{k}_v = 1;")
             elif name == "ReduceMin":
-                L.append(f"{T} r{k}_v = kun::inf<{T}>();")
+                L.append(f"{T} r{k}_v = kun::inf<{T}>(); bool r{k}_n = false;")
             elif name == "ReduceMax":
-                L.append(f"{T} r{k}_v = -kun::inf<{T}>();")
+                L.append(f"{T} r{k}_v = -kun::inf<{T}>(); bool r{k}_n = false;")
             elif name in ("ReduceArgMax", "ReduceArgMin"):
                 sgn = "-" if name == "ReduceArgMax" else ""
-                L.append(f"{T} r{k}_v = {sgn}kun::inf<{T}>(), r{k}_i = 0;")
+                L.append(f"{T} r{k}_v = {sgn}kun::inf<{T}>(); int r{k}_i = 0; bool r{k}_n = false;")
             elif name == "ReduceRank":
                 src = _rank_copy_source(r)
                 if src is None:
                     L.append(f"const {T} r{k}_cur = {self.v(r.inputs[1])};")
-                    L.append(f"{T} r{k}_lt = 0, r{k}_eq = 0;")
+                    L.append(f"const {T} r{k}_0 = 0; int r{k}_lt = 0, r{k}_eq = 0; bool r{k}_n = r{k}_cur != r{k}_cur;")
                 else:
                     # the reference copy-constructs this rank from `src`
                     # (see _rank_copy_source): it compares against src's
@@ -506,7 +506,8 @@ class _Lowering:
                     if src not in have or root.inputs[1] not in have:
                         raise RuntimeError("HIP emitter: a rank of a rank whose values sit in another kernel")
                     L.append(f"const {T} r{k}_cur = {self.v(root.inputs[1])};")
-                    L.append(f"{T} r{k}_lt = {self.v(src)} - {T}(0.5), r{k}_eq = 0;")
+                    L.append(f"const {T} r{k}_0 = {self.v(src)} - {T}(0.5); int r{k}_lt = 0, r{k}_eq = 0; "
+                             f"bool r{k}_n = r{k}_cur != r{k}_cur;")
             elif name == "ReduceDecayLinear":
                 rw = r.attrs["window"]
                 L.append(f"const {T} r{k}_step = ({T})(1.0 / ((1.0 + {rw}) * {rw} / 2));")
@@ -522,12 +523,16 @@ class _Lowering:
             name = r.__class__.__name__
             if name == "ReduceAdd" and self.fin:
                 L.append(f"v{k} = ({T})r{k}_v;")
-            elif name in ("ReduceAdd", "ReduceMul", "ReduceMin", "ReduceMax", "ReduceDecayLinear"):
+            elif name in ("ReduceAdd", "ReduceMul", "ReduceDecayLinear"):
                 L.append(f"v{k} = r{k}_v;")
+            elif name in ("ReduceMin", "ReduceMax"):
+                L.append(f"v{k} = r{k}_n ? kun::qnan<{T}>() : r{k}_v;")
             elif name in ("ReduceArgMax", "ReduceArgMin"):
-                L.append(f"v{k} = r{k}_i;")
+                L.append(f"v{k} = r{k}_n ? kun::qnan<{T}>() : ({T})r{k}_i;")
             elif name == "ReduceRank":
-                L.append(f"v{k} = r{k}_lt + (r{k}_eq + {T}(1.0)) / {T}(2.0);")
+                # exact whole and half numbers in any order
+                L.append(f"v{k} = r{k}_n ? kun::qnan<{T}>() : "
+                         f"r{k}_0 + (({T})r{k}_lt + {T}(0.5) * ({T})(r{k}_eq + 1));")
             L.extend(self.after_value(k))
         return pre, w, body_lines, L, sorted(seen)
 
@@ -547,19 +552,22 @@ class _Lowering:
                          f"r{k}_c = (t - r{k}_v) - y; r{k}_v = t; }}")
             elif name == "ReduceMul":
                 L.append(f"  r{k}_v = r{k}_v * {x};")
+            # The reference turns a result NaN at the first missing value;
+            # here the loop only notes that there was one (a compare, and an
+            # or of scalar masks), and the end selects. Positions and counts
+            # are integers, a count being a compare and an add with carry.
+            # Instructions an element: extremes 4 -> 3, their positions 7 ->
+            # 4, ranks 8 -> 5.
             elif name in ("ReduceMin", "ReduceMax"):  # Ops.hpp:487-505
                 fn = "vmin" if name == "ReduceMin" else "vmax"
-                L.append(f"  r{k}_v = (r{k}_v != r{k}_v || {x} != {x}) ? kun::qnan<{T}>() : kun::{fn}(r{k}_v, {x});")
+                L.append(f"  r{k}_n = r{k}_n || {x} != {x}; r{k}_v = kun::{fn}(r{k}_v, {x});")
             elif name in ("ReduceArgMax", "ReduceArgMin"):  # Ops.hpp:566-596
                 cmp = f"r{k}_v < {x}" if name == "ReduceArgMax" else f"r{k}_v > {x}"
-                L.append(f"  {{ const bool nn = (r{k}_v != r{k}_v) || ({x} != {x}); const bool c = {cmp};"
-                         f" r{k}_v = c ? {x} : r{k}_v; r{k}_v = nn ? kun::qnan<{T}>() : r{k}_v;"
-                         f" r{k}_i = c ? ({T})iter : r{k}_i; r{k}_i = nn ? kun::qnan<{T}>() : r{k}_i; }}")
+                L.append(f"  {{ const bool c = {cmp}; r{k}_n = r{k}_n || {x} != {x};"
+                         f" r{k}_v = c ? {x} : r{k}_v; r{k}_i = c ? iter : r{k}_i; }}")
             elif name == "ReduceRank":  # Ops.hpp:598-616
-                L.append(f"  {{ const bool nn = (r{k}_cur != r{k}_cur) || ({x} != {x});"
-                         f" r{k}_lt = nn ? kun::qnan<{T}>() : r{k}_lt;"
-                         f" r{k}_lt = ({x} < r{k}_cur) ? r{k}_lt + {T}(1.0) : r{k}_lt;"
-                         f" r{k}_eq = ({x} == r{k}_cur) ? r{k}_eq + {T}(1.0) : r{k}_eq; }}")
+                L.append(f"  r{k}_n = r{k}_n || {x} != {x}; r{k}_lt += {x} < r{k}_cur ? 1 : 0;"
+                         f" r{k}_eq += {x} == r{k}_cur ? 1 : 0;")
             elif name == "ReduceDecayLinear":  # Ops.hpp:507-520
                 L.append(f"  r{k}_v = kun::fma({x}, r{k}_w, r{k}_v); r{k}_w = r{k}_w + r{k}_step;")
         return L

@@ -55,7 +55,8 @@ void run_graph_device_noalloc(Executor &ex, const KunModuleDesc *m, const NameMa
     std::lock_guard<std::mutex> g(ex.mu);
     HIPCHECK(hipSetDevice(ex.device));
     if (!st) st = ex.stream;
-    const BatchLayout lay = batch_layout(m, S, L, ex.policy_for(m, S, L), (int)ex.lanes.size());
+    // planned for one lane, as it runs: scratch is reused along launch order
+    const BatchLayout lay = batch_layout(m, S, L, ex.policy_for(m, S, L), 1);
     if (lay.bytes > (size_t)KUN_NOALLOC_SCRATCH_BYTES)
         throw Error("kunRunGraphDeviceNoAlloc: this run needs " + std::to_string(lay.bytes) +
                     " bytes of device scratch, more than the " + std::to_string((size_t)KUN_NOALLOC_SCRATCH_BYTES) +

@@ -560,7 +560,9 @@ void plan_nodes(const KunModuleDesc *m, size_t S, size_t L, int lanes, BatchLayo
             } else {
                 if (writer[sd.in[0]] >= 0) nd.deps.push_back(writer[sd.in[0]]);
                 writer[sd.out[0]] = id;
-                nd.est = 10.0 + (double)L * (sd.kind == KUN_STAGE_RANK ? 0.18 : 0.12) * (double)S / 8192.0;
+                // 37 / 27 us for 1024 rows of 8192 floats; doubles twice that
+                nd.est = 8.0 + (double)L * (sd.kind == KUN_STAGE_RANK ? 0.03 : 0.02) * (double)S / 8192.0 *
+                                   (elem_size(m) == 8 ? 2.0 : 1.0);
             }
             std::sort(nd.deps.begin(), nd.deps.end());
             nd.deps.erase(std::unique(nd.deps.begin(), nd.deps.end()), nd.deps.end());
@@ -570,6 +572,7 @@ void plan_nodes(const KunModuleDesc *m, size_t S, size_t L, int lanes, BatchLayo
     }
     // list scheduling in topological order
     std::vector<double> lane_free(std::max(1, lanes), 0.0), finish(lay.nodes.size(), 0.0);
+    double sum = 0, full = 0, span = 0;
     for (size_t n = 0; n < lay.nodes.size(); n++) {
         BatchLayout::Node &nd = lay.nodes[n];
         double ready = 0;
@@ -592,14 +595,27 @@ void plan_nodes(const KunModuleDesc *m, size_t S, size_t L, int lanes, BatchLayo
         nd.lane = best;
         finish[n] = best_start + nd.est;
         lane_free[best] = finish[n];
+        sum += nd.est;
+        // a workgroup a row: 256 rows occupy every CU
+        if (m->stages[nd.stage].kind != KUN_STAGE_TS && L >= 256) full += nd.est;
+        span = std::max(span, finish[n]);
     }
+    // The fork, the events and the join of the lanes cost about 35 us, and
+    // kernels that fill the chip gain nothing side by side: where the lanes
+    // would save no more than their cost, one lane takes every kernel (4
+    // kernels of 64 x 260: 46 us against 79; Rank and Scale of two inputs
+    // over 1024 rows of 8192 floats: 128 us against 153, over 750 rows of
+    // 5003 doubles 143 against 163).
+    if (sum - std::max(span, full) < 30.0)
+        for (auto &nd : lay.nodes) nd.lane = 0;
 }
 
 // Enqueue every kernel of a batch module; dev[b] are device pointers, arena
 // the scratch described by `lay`. Nodes run on the executor's lanes (HIP
-// streams) as planned by plan_nodes; a node waits through events for its
-// dependencies on other lanes, every lane waits for `st` at the start and
-// `st` waits for every lane at the end.
+// streams) as planned by plan_nodes, or on `st` itself where the plan keeps
+// to one lane; a node waits through events for its dependencies on other
+// lanes, every lane the plan uses waits for `st` at the start and `st` waits
+// for it at the end.
 void enqueue_batch_serial(const KunModuleDesc *m, const std::vector<void *> &dev, const BatchLayout &lay,
                           char *arena, size_t S, size_t T, size_t start, size_t L, hipStream_t st, Executor *prof) {
     if (L == 0) return;
@@ -627,16 +643,23 @@ void enqueue_batch(Executor &ex, const KunModuleDesc *m, const std::vector<void 
         w.sync_lanes = nl;
     }
     ex.ensure_stage_events((int)lay.nodes.size());
-    HIPCHECK(hipEventRecord(ex.fork, st));
-    for (int l = 0; l < nl; l++) HIPCHECK(hipStreamWaitEvent(ex.lanes[l], ex.fork, 0));
+    std::vector<char> used(nl, 0);
+    for (const auto &nd : lay.nodes) used[nd.lane % nl] = 1;
+    const bool alone = std::count(used.begin(), used.end(), 1) <= 1;
+    if (!alone) {
+        HIPCHECK(hipEventRecord(ex.fork, st));
+        for (int l = 0; l < nl; l++)
+            if (used[l]) HIPCHECK(hipStreamWaitEvent(ex.lanes[l], ex.fork, 0));
+    }
     for (size_t n = 0; n < lay.nodes.size(); n++) {
         const auto &nd = lay.nodes[n];
-        hipStream_t ls = ex.lanes[nd.lane % nl];
+        hipStream_t ls = alone ? st : ex.lanes[nd.lane % nl];
         for (int d : lay.sync.waits[n]) HIPCHECK(hipStreamWaitEvent(ls, ex.stage_done[d], 0));
         enqueue_node(m, nd.stage, nd.kern, dev, lay, arena, S, T, start, L, ls, prof);
         if (lay.sync.record[n]) HIPCHECK(hipEventRecord(ex.stage_done[n], ls));
     }
     for (int l = 0; l < nl; l++) {
+        if (alone || !used[l]) continue;
         HIPCHECK(hipEventRecord(ex.lane_done[l], ex.lanes[l]));
         HIPCHECK(hipStreamWaitEvent(st, ex.lane_done[l], 0));
     }

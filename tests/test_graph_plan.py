@@ -127,3 +127,19 @@ def test_module_cache_key_changes_with_each_load():
     assert L.kunModuleLoadSerial(a) != L.kunModuleLoadSerial(b)
     L.kunUnloadLibrary(lib2)
     L.kunUnloadLibrary(lib1)
+
+
+@pytest.mark.parametrize("name,stocks,days,one", [
+    ("simple_f32", 64, 260, True),     # four short kernels
+    ("cs_f32", 8192, 1024, True),      # every kernel fills the chip
+    ("cs_f32", 8, 255, True),          # too few rows to fill it, too short to split
+    ("cs_f64", 16384, 200, False),     # the same with long rows: lanes pay
+    ("ops_f32", 200, 100, False),
+    ("cfg2_f32", 8192, 1024, False),
+])
+def test_runs_keep_to_one_lane_where_lanes_save_nothing(name, stocks, days, one):
+    _, mod = catalog.load(name)
+    text = kr.describeGraphBatch([(mod, stocks, days, 0, days)])
+    _, dag = parse(text)
+    assert (len({lane for _, _, lane, _ in dag[0].values()}) == 1) == one
+    check_graph(text, [mod])

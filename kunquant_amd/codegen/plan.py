@@ -229,8 +229,6 @@ def plan_stage(ops: List[OpBase], force_seq: bool = False) -> StagePlan:
     if len(unit_of) != len(ops):
         return _single_level(ops, "unscheduled ops")
     lvl: Dict[int, Optional[int]] = {}
-    # units on a sequential level that depend on a sorted window of that level
-    on_sorted: Set[int] = set()
     for u, members in enumerate(units):
         head = members[0]
         if len(members) == 1 and is_source(head):
@@ -243,16 +241,8 @@ def plan_stage(ops: List[OpBase], force_seq: bool = False) -> StagePlan:
                 if v != u and lvl[v] is not None:
                     m = max(m, lvl[v])
         name = head.__class__.__name__
-        after_sorted = m % 2 == 1 and any(unit_of[inp] in on_sorted and lvl[unit_of[inp]] == m
-                                          for o in members for inp in o.inputs if unit_of[inp] != u)
         if name in REC_OPS:
             lvl[u] = m if m % 2 == 1 else m + 1
-            # a recurrence over a sorted window's value takes the next
-            # sequential level: the window can then run row-chunked, its
-            # value handed over through memory (17 of the 150-factor graph's
-            # 48 quantiles feed a rolling sum or regression)
-            if after_sorted and name != "SkipListState":
-                lvl[u] = m + 2
         elif name in BOUND_OPS:
             state = lvl[unit_of[head.inputs[0]]]
             if state is None or m > state:
@@ -262,8 +252,6 @@ def plan_stage(ops: List[OpBase], force_seq: bool = False) -> StagePlan:
             lvl[u] = m if m % 2 == 0 else m + 1
         else:
             lvl[u] = m
-        if name == "SkipListState" or (after_sorted and lvl[u] == m):
-            on_sorted.add(u)
     # Sequential levels walk every row on one lane per stock, so they keep
     # only what their recurrences need: a unit on a sequential level that no
     # recurrence (or state consumer) of the level depends on moves to the

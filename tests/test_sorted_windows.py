@@ -91,41 +91,3 @@ def test_only_pure_windows_are_split():
                 if op.__class__.__name__ == "SkipListState":
                     assert is_window_sorted(op) == (op.inputs[0].attrs["window"] == 9)
     assert split == {"good": True, "other": False, "ema": False}
-
-
-@pytest.mark.parametrize("dtype", ["float", "double"])
-def test_a_recurrence_over_a_quantile_leaves_it_split(dtype):
-    """The recurrence takes a later sequential level and reads the quantile's
-    value from memory; one the quantile itself follows stays before it."""
-    w = 5
-    b = Builder()
-    with b:
-        a = Input("a")
-        q = WindowedQuantile(a, w, 0.4)
-        Output(ExpMovingAvg(q * 2, 6), "ema_of_q")
-        Output(WindowedQuantile(ExpMovingAvg(q, 3), w, 0.7), "q_of_ema_of_q")
-        Output(ExpMovingAvg(a, 6), "ema")
-    m = compileit(Function(b.ops), f"recsorted_{dtype}", input_layout="TS", output_layout="TS", dtype=dtype,
-                  options={"no_fast_stat": "no_warn"})
-    splits = []
-    for st in m.stages:
-        plan = stage_plan(m, st)
-        for level in plan.levels:
-            for c in level.comps:
-                for op in c.ops:
-                    if op.__class__.__name__ == "SkipListState" and is_window_sorted(op):
-                        splits.append(rows_splittable(plan, c))
-    assert splits and all(splits)
-    S, T, start = 9, 60, 3
-    L = T - start
-    a = _rows(T, S, np.float32 if dtype == "float" else np.float64)
-    exp = OracleProgram(program_text(m)).run({"a": a}, S, T, start, L, nthreads=2, temps=True)
-    emu = EmuModule(m)
-    for st in m.stages:
-        for chunk in (0, 1, w, 16):
-            got = {"a": a, **exp}
-            for buf in st.out_bufs:
-                got[buf.name] = np.full_like(exp[buf.name], 12345.0)
-            emu.run_stage(st.idx, got, S, T, start, L, chunk)
-            for buf in st.out_bufs:
-                assert_bit_exact(got[buf.name], exp[buf.name], f"{buf.name} chunk {chunk}")

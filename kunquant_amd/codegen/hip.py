@@ -95,6 +95,10 @@ ROW_BARRIER = 0x9C
 # than two: 2 / 3 / 4 rows ran the 100-factor fp32 graph in 26.6 / 25.9 /
 # 25.4 ms (row-chunked kernels alone 18.8 / 17.6 / 17.1)
 INTERLEAVE_MIN, INTERLEAVE_MAX = 4, 4
+# rows of a group where more would spill more ring slots to scratch columns
+# (2 of the 100-factor graph's 171 such components): what a run needs of
+# device memory, and the no-allocation entry's limit, stay where they are
+INTERLEAVE_SPILL = 2
 
 _BIN = {"Add": "+", "Sub": "-", "Mul": "*", "Div": "/"}
 _CMP = {"GreaterThan": ">", "GreaterEqual": ">=", "LessThan": "<", "LessEqual": "<=", "Equals": "=="}
@@ -792,6 +796,19 @@ class StageEmitter(_Lowering):
         return "\n".join(tick) + "\n\n" + "\n".join(init)
 
 
+def _spilled_slots(needs: List[int], rows: int, cap: int) -> int:
+    """Ring slots of a component that do not fit `cap` slots of LDS, for
+    groups of `rows` rows; needs: each ring's largest offset."""
+    n_lds = n = 0
+    for need in needs:
+        slots = need + rows
+        if n_lds + slots <= cap:
+            n_lds += slots
+        else:
+            n += slots
+    return n
+
+
 class CompEmitter(_Lowering):
     """One component of one level of a batch time-series stage.
 
@@ -845,11 +862,16 @@ class CompEmitter(_Lowering):
             p = min(max(p, INTERLEAVE_MIN), INTERLEAVE_MAX)
             p = max(1, min(p, PREFETCH_REGS // max(1, len(self.srcs) + len(self.lags))))
             self.interleave = p if p > 1 else 0
+        cap = lds_budget_for(module, lds_budget, kind == SEQ) // (self.esz * TS_BLOCK)
+        if self.interleave > INTERLEAVE_SPILL:
+            # a run's scratch columns do not grow with the rows of a group
+            needs = [ring_need[op] for op in sorted(ring_need, key=lambda o: self.idx[o])]
+            if _spilled_slots(needs, self.interleave, cap) > _spilled_slots(needs, INTERLEAVE_SPILL, cap):
+                self.interleave = INTERLEAVE_SPILL
         extra = self.interleave - 1 if self.interleave else 0
         self.ring: Dict[int, Tuple[int, int]] = {}
         self.tslot: Dict[int, int] = {}
         self.islot: Dict[int, int] = {}
-        cap = lds_budget_for(module, lds_budget, kind == SEQ) // (self.esz * TS_BLOCK)
         n_lds = 0
         spilled = []
         for op in sorted(ring_need, key=lambda o: self.idx[o]):

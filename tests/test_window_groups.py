@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 from emu.emu import EmuModule
+from kunquant_amd.codegen import hip
 from kunquant_amd.codegen.program import program_text
 from kunquant_amd.Driver import compileit
 from kunquant_amd.Op import Builder, Input, Output
@@ -63,3 +64,30 @@ def test_groups_equal_the_oracle(dtype, w, lds):
             emu.run_stage(st.idx, got, S, T, start, L, chunk)
             for b in st.out_bufs:
                 assert_bit_exact(got[b.name], exp[b.name], f"{b.name} chunk {chunk}")
+
+
+@pytest.mark.parametrize("dtype", ["float", "double"])
+@pytest.mark.parametrize("lds", [None, 1024, 3072, 4096, 8192])
+def test_scratch_does_not_grow_with_the_rows_of_a_group(dtype, lds, monkeypatch):
+    """Groups of four rows need three more slots a ring; a component whose
+    rings would then spill more than with two rows keeps to two."""
+    m = compileit(_graph(37), f"spill_{dtype}_{lds}", input_layout="TS", output_layout="TS", dtype=dtype,
+                  options={"no_fast_stat": True})
+
+    def comps():
+        out = []
+        for st in m.stages:
+            plan = hip.stage_plan(m, st)
+            for level in plan.levels:
+                for c in level.comps:
+                    out.append(hip.CompEmitter(m, st, plan, c, level.kind, lds))
+        return [e for e in out if e.interleave]
+
+    now = comps()
+    monkeypatch.setattr(hip, "INTERLEAVE_MIN", 2)
+    monkeypatch.setattr(hip, "INTERLEAVE_MAX", 2)
+    two = comps()
+    assert len(now) == len(two) > 0
+    for e, t in zip(now, two):
+        assert t.interleave == 2 and e.interleave in (2, 4)
+        assert e.spill_bytes == t.spill_bytes if e.interleave == 2 else e.spill_bytes <= t.spill_bytes

@@ -370,8 +370,10 @@ static void plan_slots(const KunModuleDesc *m, size_t S, size_t L, size_t base, 
             for (int r = 0; r < kd.nmat_reads; r++) rd(mb + kd.mat_reads[r]);
             for (int w = 0; w < kd.nmat_writes; w++) wr(mb + kd.mat_writes[w]);
         } else {
-            if (is_temp(sd.in[0])) rd(sd.in[0]);
-            if (is_temp(sd.out[0])) wr(sd.out[0]);
+            for (int j = 0; j < sd.nin; j++)
+                if (is_temp(sd.in[j])) rd(sd.in[j]);
+            for (int j = 0; j < sd.nout; j++)
+                if (is_temp(sd.out[j])) wr(sd.out[j]);
         }
     }
     std::vector<int> slot_of(nval, -1), occupant;
@@ -558,8 +560,11 @@ void plan_nodes(const KunModuleDesc *m, size_t S, size_t L, int lanes, BatchLayo
                 nd.est = kd.kind == KUN_KERNEL_PAR ? 5.0 + work * 4.0 / (1024.0 * 2400.0 * 0.4)
                                                    : 20.0 + (double)L * seq * 8.0 / 2400.0;
             } else {
-                if (writer[sd.in[0]] >= 0) nd.deps.push_back(writer[sd.in[0]]);
-                writer[sd.out[0]] = id;
+                // Rank and Scale have one input and one output, a generic
+                // cross-sectional op as many as its body takes
+                for (int j = 0; j < sd.nin; j++)
+                    if (writer[sd.in[j]] >= 0) nd.deps.push_back(writer[sd.in[j]]);
+                for (int j = 0; j < sd.nout; j++) writer[sd.out[j]] = id;
                 // 37 / 27 us for 1024 rows of 8192 floats; doubles twice that
                 nd.est = 8.0 + (double)L * (sd.kind == KUN_STAGE_RANK ? 0.03 : 0.02) * (double)S / 8192.0 *
                                    (elem_size(m) == 8 ? 2.0 : 1.0);

@@ -370,6 +370,21 @@ def generic_cs_graph(K=None):
     return K.Function(b.ops)
 
 
+def generic_pair_graph(K=None):
+    """Generic cross-sectional ops whose two inputs are both computed: by
+    other cross-sectional ops, by a time-series stage and by each other."""
+    K = K or native()
+    b = K.Builder()
+    with b:
+        a, bb, c = K.Input("a"), K.Input("b"), K.Input("c")
+        d = K.DiffWithWeightedSum(K.Rank(a), K.Rank(c))
+        e = K.DiffWithWeightedSum(K.Scale(bb), K.Rank(bb))
+        K.Output(d, "ranks")
+        K.Output(K.DiffWithWeightedSum(K.WindowedAvg(d, 5), K.Scale(a - c)), "avg_scale")
+        K.Output(K.DiffWithWeightedSum(d, e), "chain")
+    return K.Function(b.ops)
+
+
 def cross_section_graph(K=None):
     """Rank and Scale straight off the inputs (cross-sectional kernel checks)."""
     K = K or native()

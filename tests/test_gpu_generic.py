@@ -6,6 +6,8 @@ DiffWithWeightedSum(a - b, c), its 5-row average and its rank.
     (tests/golden/ref_generic_f32.npz) bit for bit;
   * STs fp64 module: equal to the oracle bit for bit;
   * stream module: tick by tick equal to the reference's batch outputs;
+  * generic ops with two computed inputs (fp32 TS): equal to the oracle bit for
+    bit as a plain run, a batch of jobs, a graph of them and without allocations;
   * session pools refuse the module (the body runs in stream contexts).
 
 Bar: bit-exact (NaN positions equal, NaN payload bits ignored)."""
@@ -18,6 +20,7 @@ from kunquant_amd.codegen.program import program_text
 from kunquant_amd.runner import KunRunner as kr
 from kunquant_amd.workloads import catalog
 from oracle.kun_oracle import OracleProgram
+from tests.test_zz_no_alloc import _no_alloc, capi  # noqa: F401 (a fixture)
 
 pytestmark = pytest.mark.gpu
 
@@ -77,6 +80,40 @@ def test_stream_module_matches_reference(executor, golden):
         st.run()
         for k in outs:
             assert _same(st.getCurrentBuffer(h[k]), outs[k][t]), (k, t)
+
+
+@pytest.mark.parametrize("S,T", [(64, 40), (800, 500)])
+def test_two_computed_inputs_match_oracle(executor, capi, S, T):
+    torch = pytest.importorskip("torch")
+    _, mod = catalog.load("generic_pair_f32")
+    prog = OracleProgram(program_text(catalog.module_ir("generic_pair_f32")))
+    rng = np.random.default_rng(S + T)
+    jobs, exp = [], []
+    for _ in range(2):
+        ins = {k: rng.standard_normal((T, S)).astype(np.float32) for k in ("a", "b", "c")}
+        ins["c"][T // 2, 1] = np.nan
+        dev = {k: torch.from_numpy(v).cuda() for k, v in ins.items()}
+        out = {k: torch.empty((T, S), device="cuda") for k in mod.getOutputNames()}
+        jobs.append((mod, dev, out))
+        exp.append(prog.run(ins, S, T, 0, T, nthreads=4))
+        got = kr.runGraph(executor, mod, ins, 0, T)
+        assert not [k for k in exp[-1] if not _same(got[k], exp[-1][k])]
+    tuples = [(m, {k: v.data_ptr() for k, v in {**i, **o}.items()}, S, T, 0, T) for m, i, o in jobs]
+    graph = kr.BatchGraph(executor, tuples)
+    ways = dict(batch=lambda: kr.runGraphBatchDevice(executor, tuples), graph=graph.launch, replay=graph.launch,
+                device=lambda: [kr.runGraphDevice(executor, *t) for t in tuples],
+                no_alloc=lambda: [_no_alloc(capi, executor, m, t[1], S, T) for m, t in zip((mod, mod), tuples)])
+    for way, call in ways.items():
+        for _, _, out in jobs:
+            for v in out.values():
+                v.fill_(12345.0)
+        torch.cuda.synchronize()
+        call()
+        executor.synchronize()
+        torch.cuda.synchronize()
+        for (_, _, out), e in zip(jobs, exp):
+            bad = [k for k in e if not _same(out[k].cpu().numpy(), e[k])]
+            assert not bad, (way, bad)
 
 
 def test_pool_refuses_generic_stage(executor):

@@ -31,7 +31,7 @@ import numpy as np
 
 from ..Driver import BUF_INPUT, BUF_TEMP, ModuleIR, STAGE_GENERIC, STAGE_TS
 from ..Op import ConstantOp, ForeachBackWindow, Input, OpBase, Output, ReductionOp
-from .plan import PAR, SEQ, Component, StagePlan, plan_stage, rows_splittable
+from .plan import PAR, SEQ, Component, StagePlan, is_window_sorted, plan_stage, rows_splittable
 from .program import literal, program_text
 from .wire import wire_table
 
@@ -1177,7 +1177,8 @@ class CompEmitter(_Lowering):
             elif name == "SkipListState":
                 w = op.attrs["window"]
                 if k in self.sorted_regs:
-                    L.append(f"kun::SortedWinR<{T}, {w}, {'true' if self.sorted_regs[k] else 'false'}> st{k};")
+                    win = "SortedWinR" if is_window_sorted(op) else "SortedAnyR"
+                    L.append(f"kun::{win}<{T}, {w}, {'true' if self.sorted_regs[k] else 'false'}> st{k};")
                     continue
                 ts, is_ = self.tslot[k], self.islot[k]
                 L.append(f"kun::SortedWin<{T}, {w}> st{k}; st{k}.init(stT + (size_t)({ts - self.lds_t}) * cst, "

@@ -341,27 +341,65 @@ template <typename T, int W> struct SortedWin {
     }
 };
 
-// The same sorted window held in registers (batch kernels): W slots that are
-// always all in use, a missing value being a slot of +inf at its place in the
-// order of arrival. One row takes the oldest arrival out and puts the newest
-// in, in one pass of compile-time slots. Equal values, the empty slots among
-// them, stand in order of arrival, so the first of them is the one to leave
-// and a new one goes after the last (SortedWin's order); quantities of the
-// window are read only while all W values are there (n == W), when no empty
-// slot is left. IDX keeps the row indices (SkipListArgMin).
+// A sorted window held in registers (batch kernels): SLOTS compile-time slots,
+// and what is read from them. IDX keeps the row indices (SkipListArgMin).
+template <typename T, int W, int SLOTS, bool IDX> struct SortedRegs {
+    T v[SLOTS];
+    int32_t ix[IDX ? SLOTS : 1];
+    int n = 0, last = 0;
+    __device__ __forceinline__ explicit SortedRegs(T fill) {
+#pragma unroll
+        for (int k = 0; k < SLOTS; k++) v[k] = fill;
+#pragma unroll
+        for (int k = 0; k < (IDX ? SLOTS : 1); k++) ix[k] = 0;
+    }
+    __device__ __forceinline__ T at(int i) const {
+        T r = T(0);
+#pragma unroll
+        for (int k = 0; k < SLOTS; k++) r = k == i ? v[k] : r;
+        return r;
+    }
+    __device__ __forceinline__ T quantile(T q, long) const {
+        if (n != W) return qnan<T>();
+        T f = q * (T)(n - 1);
+        int i = (int)f;
+        if ((T)i == f) return at(i);
+        double lo = (double)at(i), hi = (double)at(i + 1);
+        return (T)(lo + (hi - lo) * (double)(f - (T)i));
+    }
+    __device__ __forceinline__ T rank(T cur, long) const {
+        if (n != W) return qnan<T>();
+        int lt = 0;
+#pragma unroll
+        for (int k = 0; k < W; k++) lt += v[k] < cur ? 1 : 0;
+        double r = last + 1, rmin = lt + 1;
+        r = (((r * (r + 1) / 2) - ((rmin - 1) * rmin / 2)) / (r - rmin + 1));
+        return (T)r;
+    }
+    __device__ __forceinline__ T vmin_(long) const { return n != W ? qnan<T>() : v[0]; }
+    __device__ __forceinline__ T vmax_(long) const { return n != W ? qnan<T>() : v[W - 1]; }
+    __device__ __forceinline__ T argmin(int64_t cur_idx, long) const {
+        if (n != W) return qnan<T>();
+        return (T)(int64_t)(ix[0] + n - cur_idx);
+    }
+};
+
+// The window whose leaving value is the one that entered W rows earlier: W
+// slots that are always all in use, a missing value being a slot of +inf at
+// its place in the order of arrival. One row takes the oldest arrival out and
+// puts the newest in, in one pass of compile-time slots. Equal values, the
+// empty slots among them, stand in order of arrival, so the first of them is
+// the one to leave and a new one goes after the last (SortedWin's order);
+// quantities of the window are read only while all W values are there
+// (n == W), when no empty slot is left.
 //
 // 2 compares and 3 selects a slot and row; searching, shifting and storing
-// in separate passes with a count of used slots took about four times that.
-template <typename T, int W, bool IDX> struct SortedWinR {
-    T v[W];
-    int32_t ix[IDX ? W : 1];
-    int n = 0, last = 0;
-    __device__ __forceinline__ SortedWinR() {
-#pragma unroll
-        for (int k = 0; k < W; k++) v[k] = inf<T>();
-#pragma unroll
-        for (int k = 0; k < (IDX ? W : 1); k++) ix[k] = 0;
-    }
+// in separate passes with a count of used slots (SortedAnyR) took about four
+// times that.
+template <typename T, int W, bool IDX> struct SortedWinR : SortedRegs<T, W, W, IDX> {
+    using B = SortedRegs<T, W, W, IDX>;
+    using B::ix, B::last, B::n, B::v;
+    __device__ __forceinline__ SortedWinR() : B(inf<T>()) {}
     __device__ __forceinline__ void step(T old, T cur, int32_t index, long) {
         n += (cur == cur ? 1 : 0) - (old == old ? 1 : 0);
         const T o = old == old ? old : inf<T>();
@@ -389,34 +427,51 @@ template <typename T, int W, bool IDX> struct SortedWinR {
         }
         last = pos;
     }
-    __device__ __forceinline__ T at(int i) const {
-        T r = T(0);
+};
+
+// The window of a state whose leaving value may be any value, in the window
+// or not (any `oldvalue` but the entering value W rows ago): searched for,
+// and taken out only where it is found, as SortedWin does. A window the
+// leaving value is missing from holds more than W values; the largest past
+// W + 1 are lost.
+template <typename T, int W, bool IDX> struct SortedAnyR : SortedRegs<T, W, W + 1, IDX> {
+    using B = SortedRegs<T, W, W + 1, IDX>;
+    using B::ix, B::last, B::n, B::v;
+    __device__ __forceinline__ SortedAnyR() : B(T(0)) {}
+    __device__ __forceinline__ void step(T old, T cur, int32_t index, long) {
+        if (old == old) {
+            int p = 0;
 #pragma unroll
-        for (int k = 0; k < W; k++) r = k == i ? v[k] : r;
-        return r;
-    }
-    __device__ __forceinline__ T quantile(T q, long) const {
-        if (n != W) return qnan<T>();
-        T f = q * (T)(n - 1);
-        int i = (int)f;
-        if ((T)i == f) return at(i);
-        double lo = (double)at(i), hi = (double)at(i + 1);
-        return (T)(lo + (hi - lo) * (double)(f - (T)i));
-    }
-    __device__ __forceinline__ T rank(T cur, long) const {
-        if (n != W) return qnan<T>();
-        int lt = 0;
+            for (int k = 0; k <= W; k++) p += (k < n && v[k] < old) ? 1 : 0;
+            bool found = false;
 #pragma unroll
-        for (int k = 0; k < W; k++) lt += v[k] < cur ? 1 : 0;
-        double r = last + 1, rmin = lt + 1;
-        r = (((r * (r + 1) / 2) - ((rmin - 1) * rmin / 2)) / (r - rmin + 1));
-        return (T)r;
-    }
-    __device__ __forceinline__ T vmin_(long) const { return n != W ? qnan<T>() : v[0]; }
-    __device__ __forceinline__ T vmax_(long) const { return n != W ? qnan<T>() : v[W - 1]; }
-    __device__ __forceinline__ T argmin(int64_t cur_idx, long) const {
-        if (n != W) return qnan<T>();
-        return (T)(int64_t)(ix[0] + n - cur_idx);
+            for (int k = 0; k <= W; k++) found = found || (k == p && k < n && v[k] == old);
+            if (found) {
+#pragma unroll
+                for (int k = 0; k < W; k++) {
+                    v[k] = k >= p ? v[k + 1] : v[k];
+                    if (IDX) ix[k] = k >= p ? ix[k + 1] : ix[k];
+                }
+                n--;
+            }
+        }
+        if (cur == cur) {
+            int p = 0;
+#pragma unroll
+            for (int k = 0; k <= W; k++) p += (k < n && v[k] <= cur) ? 1 : 0;
+#pragma unroll
+            for (int k = W; k > 0; k--) {
+                v[k] = k > p ? v[k - 1] : v[k];
+                if (IDX) ix[k] = k > p ? ix[k - 1] : ix[k];
+            }
+#pragma unroll
+            for (int k = 0; k <= W; k++) {
+                v[k] = k == p ? cur : v[k];
+                if (IDX) ix[k] = k == p ? index : ix[k];
+            }
+            n++;
+            last = p;
+        }
     }
 };
 

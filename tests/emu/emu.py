@@ -6,6 +6,7 @@ are run lane by lane (tests/emu/kun_emu.cpp). Tests compare the result of
 every time-series stage with the oracle's value of the same buffers, so the
 emitter, the kernel plan and the row chunking are checked without a GPU."""
 import ctypes
+import hashlib
 import os
 import subprocess
 
@@ -16,13 +17,24 @@ ROOT = os.path.dirname(os.path.dirname(HERE))
 BUILD = os.path.join(HERE, "_build")
 
 
+def _headers() -> str:
+    h = hashlib.sha256()
+    for d in (os.path.join(HERE, "include", "hip"), os.path.join(ROOT, "kunquant_amd", "csrc"), HERE):
+        for f in sorted(os.listdir(d)):
+            if f.endswith((".h", ".hpp", ".cpp")):
+                with open(os.path.join(d, f), "rb") as fh:
+                    h.update(fh.read())
+    return h.hexdigest()[:16]
+
+
 def build(module_ir, lds_budget=None) -> str:
     from kunquant_amd.codegen.hip import emit_module, ident
     os.makedirs(BUILD, exist_ok=True)
     name = ident(module_ir.name) + ("" if lds_budget is None else f"_lds{lds_budget}")
     src = os.path.join(BUILD, f"{name}.cpp")
     out = os.path.join(BUILD, f"{name}.so")
-    text = emit_module(module_ir, lds_budget)
+    # built again when the emitted source or a header it includes changes
+    text = f"// headers {_headers()}\n" + emit_module(module_ir, lds_budget)
     if os.path.exists(out) and os.path.exists(src) and open(src).read() == text:
         return out
     with open(src, "w") as f:

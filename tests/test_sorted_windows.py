@@ -91,3 +91,51 @@ def test_only_pure_windows_are_split():
                 if op.__class__.__name__ == "SkipListState":
                     assert is_window_sorted(op) == (op.inputs[0].attrs["window"] == 9)
     assert split == {"good": True, "other": False, "ema": False}
+
+
+@pytest.mark.parametrize("dtype", ["float", "double"])
+@pytest.mark.parametrize("w", [1, 2, 7, 150])
+def test_any_leaving_value_equals_the_oracle(dtype, w):
+    """States whose leaving value is not the value that entered a window ago:
+    only what is found leaves. `a` and `c` are the same series but for cells
+    missing from one of them, so that a value leaves that never entered, or
+    one that entered stays (at most one a stock: no window ever holds more
+    than w + 1 values); a lag of w + 1 holds w values only where one of them
+    is missing. In registers, and (150 rows) in scratch columns."""
+    b = Builder()
+    with b:
+        a, c = Input("a"), Input("c")
+        for name, st in (("other", SkipListState(BackRef(c, w), a, w)),
+                         ("longer", SkipListState(BackRef(a, w + 1), a, w)),
+                         ("computed", SkipListState(BackRef(c * 2, w), a * 2, w))):
+            assert not is_window_sorted(st)
+            Output(SkipListQuantile(st, 0.3), f"q_{name}")
+            Output(SkipListMin(st), f"min_{name}")
+            Output(SkipListMax(st), f"max_{name}")
+            Output(SkipListArgMin([st], []), f"argmin_{name}")
+    m = compileit(Function(b.ops), f"leaving{w}_{dtype}", input_layout="TS", output_layout="TS", dtype=dtype,
+                  options={"no_fast_stat": "no_warn"})
+    S, T = 9, 4 * w + 40
+    dt = np.float32 if dtype == "float" else np.float64
+    rng = np.random.default_rng(w)
+    x = rng.standard_normal((T, S))
+    x[:, 1] = np.round(x[:, 1] * 2)
+    a, c = x.astype(dt), x.astype(dt)
+    for s in range(S):
+        gone = rng.choice(np.arange(1, T), 3 + T // (w + 3), replace=False)
+        a[gone[1:], s] = np.nan             # leaves without having entered
+        if s % 3:
+            c[:, s] = np.where(np.isin(np.arange(T), gone[2:]), np.nan, c[:, s])
+            c[gone[0], s] = np.nan          # entered and stays
+    exp = OracleProgram(program_text(m)).run({"a": a, "c": c}, S, T, 0, T, nthreads=2, temps=True)
+    for name in ("q_other", "q_longer", "q_computed"):
+        assert np.isfinite(exp[name][T // 2:]).sum() >= 10, name
+    emu = EmuModule(m)
+    for st in m.stages:
+        for chunk in (0, 16):
+            got = {"a": a, "c": c, **exp}
+            for o in st.out_bufs:
+                got[o.name] = np.full_like(exp[o.name], 12345.0)
+            emu.run_stage(st.idx, got, S, T, 0, T, chunk)
+            for o in st.out_bufs:
+                assert_bit_exact(got[o.name], exp[o.name], f"{o.name} chunk {chunk}")

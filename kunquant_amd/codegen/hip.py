@@ -268,6 +268,12 @@ def window_loop(w: int, body: List[str], unroll: int, loads=None, fast=None, row
             + loop_code(w, body, unroll, loads) + ["}"])
 
 
+def _any_leaves(op) -> str:
+    """Template argument of kun::SortedWin: whether a value may leave that
+    did not enter a window ago."""
+    return "" if is_window_sorted(op) else ", true"
+
+
 def _flatten(segs, unroll: int, loads_of=lambda srcs: (None, None)) -> List[str]:
     L = []
     for sg in segs:
@@ -712,7 +718,7 @@ class StageEmitter(_Lowering):
                 L.append(f"  {T} acc{k} = {self.tmem(ts)};")
             elif name == "SkipListState":
                 w = op.attrs["window"]
-                L.append(f"  kun::SortedWin<{T}, {w}> st{k}; st{k}.init(stT + (size_t){ts} * A.S, "
+                L.append(f"  kun::SortedWin<{T}, {w}{_any_leaves(op)}> st{k}; st{k}.init(stT + (size_t){ts} * A.S, "
                          f"istp + (size_t){is_} * A.S, A.S);")
                 L.append(f"  st{k}.n = {self.imem(is_ + w + 1)}; st{k}.last = {self.imem(is_ + w + 2)};")
         return L
@@ -1181,7 +1187,7 @@ class CompEmitter(_Lowering):
                     L.append(f"kun::{win}<{T}, {w}, {'true' if self.sorted_regs[k] else 'false'}> st{k};")
                     continue
                 ts, is_ = self.tslot[k], self.islot[k]
-                L.append(f"kun::SortedWin<{T}, {w}> st{k}; st{k}.init(stT + (size_t)({ts - self.lds_t}) * cst, "
+                L.append(f"kun::SortedWin<{T}, {w}{_any_leaves(op)}> st{k}; st{k}.init(stT + (size_t)({ts - self.lds_t}) * cst, "
                          f"istp + (size_t){is_} * cst, cst);")
         return L
 

@@ -275,8 +275,10 @@ template <typename T> struct LinReg {
 // column-wise ([W+1][stride], LDS in batch kernels, HBM in stream kernels);
 // restates the skip-list state of Ops/Quantile.hpp:15-45. Insertion goes
 // after equal values and removal takes the first equal value, so ties keep
-// insertion order like the reference skip list.
-template <typename T, int W> struct SortedWin {
+// insertion order like the reference skip list. ANY: the leaving value may
+// be any value, not the one that entered W rows earlier; a window it is
+// missing from grows past W values, of which the W + 1 smallest are kept.
+template <typename T, int W, bool ANY = false> struct SortedWin {
     T *val;      // [W + 1][stride]
     int32_t *ix; // [W + 1][stride]
     long stride;
@@ -290,12 +292,15 @@ template <typename T, int W> struct SortedWin {
     }
     __device__ __forceinline__ T get(int k, long lane) const { return val[k * stride + lane]; }
     __device__ __forceinline__ int32_t idx(int k, long lane) const { return ix[k * stride + lane]; }
+    // values that are kept
+    __device__ __forceinline__ int used() const { return ANY && n > W + 1 ? W + 1 : n; }
     __device__ __forceinline__ void step(T old, T cur, int32_t index, long lane) {
         if (old == old) {
+            const int m = used();
             int p = 0;
-            while (p < n && get(p, lane) < old) p++;
-            if (p < n && get(p, lane) == old) {
-                for (int q = p; q < n - 1; q++) {
+            while (p < m && get(p, lane) < old) p++;
+            if (p < m && get(p, lane) == old) {
+                for (int q = p; q < m - 1; q++) {
                     val[q * stride + lane] = val[(q + 1) * stride + lane];
                     ix[q * stride + lane] = ix[(q + 1) * stride + lane];
                 }
@@ -303,14 +308,17 @@ template <typename T, int W> struct SortedWin {
             }
         }
         if (cur == cur) {
+            const int m = used();
             int p = 0;
-            while (p < n && get(p, lane) <= cur) p++;
-            for (int q = n; q > p; q--) {
+            while (p < m && get(p, lane) <= cur) p++;
+            for (int q = ANY && m > W ? W : m; q > p; q--) {
                 val[q * stride + lane] = val[(q - 1) * stride + lane];
                 ix[q * stride + lane] = ix[(q - 1) * stride + lane];
             }
-            val[p * stride + lane] = cur;
-            ix[p * stride + lane] = index;
+            if (!ANY || p <= W) {
+                val[p * stride + lane] = cur;
+                ix[p * stride + lane] = index;
+            }
             n++;
             last = p;
         }

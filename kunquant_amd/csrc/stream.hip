@@ -203,7 +203,7 @@ template <typename T, typename IT> static void wire_write(const WireView &c, Wir
                 const int32_t *last = icol<T>(st, ws.tslots, ws.islot + W + 2, S);
                 out.append((const char *)(last + s0), B * sizeof(int32_t));
                 for (size_t l = 0; l < B; l++) {
-                    const int32_t k = cnt[s0 + l];
+                    const int32_t k = std::min(cnt[s0 + l], W + 1); // values that are kept
                     out.append((const char *)&k, sizeof k);
                     for (int q = 0; q < k; q++) {
                         const double v = (double)tcol<T>(st, ws.tslot + q, S)[s0 + l];

@@ -139,3 +139,35 @@ def test_any_leaving_value_equals_the_oracle(dtype, w):
             emu.run_stage(st.idx, got, S, T, 0, T, chunk)
             for o in st.out_bufs:
                 assert_bit_exact(got[o.name], exp[o.name], f"{o.name} chunk {chunk}")
+
+
+@pytest.mark.parametrize("dtype", ["float", "double"])
+def test_windows_that_grow_keep_to_their_columns(dtype):
+    """A state whose leaving values are never in its window grows with every
+    row. In scratch columns it keeps to its own w + 1 slots: the window in the
+    next columns is that of a module without it."""
+    w, S, T = 150, 9, 600
+
+    def graph(grow):
+        b = Builder()
+        with b:
+            a, c = Input("a"), Input("c")
+            first = SkipListArgMin([SkipListState(BackRef(c, w), a, w)], [])
+            second = SkipListArgMin([SkipListState(BackRef(a, w), a, w)], [])
+            Output(second, "second")
+            Output(first + second if grow else c - second, "joint")
+        return Function(b.ops)
+
+    dt = np.float32 if dtype == "float" else np.float64
+    rng = np.random.default_rng(3)
+    a = rng.standard_normal((T, S)).astype(dt)
+    ins = {"a": a, "c": a + dt(1000)}
+    opt = dict(input_layout="TS", output_layout="TS", dtype=dtype, options={"no_fast_stat": "no_warn"})
+    exp = OracleProgram(program_text(compileit(graph(False), "g", **opt))).run(ins, S, T, 0, T)
+    m = compileit(graph(True), f"grow_{dtype}", **opt)
+    emu = EmuModule(m)
+    (st,) = m.stages
+    got = {**ins, **{o.name: np.full((T, S), 12345.0, dt) for o in st.out_bufs}}
+    emu.run_stage(st.idx, got, S, T, 0, T, 0)
+    assert_bit_exact(got["second"], exp["second"], "second")
+    assert np.isnan(got["joint"][w + 1:]).all()

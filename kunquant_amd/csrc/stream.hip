@@ -21,6 +21,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <fstream>
 #include <iterator>
 #include <limits>
@@ -60,9 +61,14 @@ struct StreamCtx {
     size_t S = 0, esz = 4, tick = 0;
     std::vector<void *> rows;       // device rows per buffer
     std::vector<void *> host_rows;  // pinned mirrors for getCurrentBuffer
-    std::vector<char> host_valid;
-    std::vector<char> wanted;       // rows read on the host since the last tick
-    std::vector<char> exposed;      // rows whose device pointer was given out
+    // Rows may be read by one thread while another runs ticks. Everything
+    // below changes under the executor's lock but `wanted`; a read or a
+    // device pointer that needs no more than what the flags already say takes
+    // none.
+    using Flags = std::vector<std::atomic<char>>;
+    Flags host_valid;
+    Flags wanted;                   // rows read on the host since the last tick (a hint)
+    Flags exposed;                  // rows whose device pointer was given out
     std::vector<void *> ticked;     // pinned: wanted rows as the last tick left them
     std::vector<char> ticked_valid;
     std::vector<void *> state;      // per stage: [state_bytes * S]
@@ -345,9 +351,7 @@ StreamCtx *stream_create(std::shared_ptr<Executor> ex, const KunModuleDesc *m, s
     HIPCHECK(hipSetDevice(ex->device));
     c->rows.resize(m->nbuf, nullptr);
     c->host_rows.resize(m->nbuf, nullptr);
-    c->host_valid.assign(m->nbuf, 0);
-    c->wanted.assign(m->nbuf, 0);
-    c->exposed.assign(m->nbuf, 0);
+    for (auto *f : {&c->host_valid, &c->wanted, &c->exposed}) StreamCtx::Flags(m->nbuf).swap(*f);
     c->ticked.assign(m->nbuf, nullptr);
     c->ticked_valid.assign(m->nbuf, 0);
     for (int b = 0; b < m->nbuf; b++) {
@@ -410,6 +414,7 @@ void stream_run(StreamCtx *c) {
     const KunModuleDesc *m = c->m;
     std::lock_guard<std::mutex> g(c->ex->mu);
     HIPCHECK(hipSetDevice(c->ex->device));
+    std::fill(c->ticked_valid.begin(), c->ticked_valid.end(), 0); // also if this tick fails
     for (int si : stage_order(m)) {
         const KunStageDesc &sd = m->stages[si];
         if (sd.kind == KUN_STAGE_TS) {
@@ -468,32 +473,33 @@ void stream_run(StreamCtx *c) {
         HIPCHECK(hipGetLastError());
     }
     HIPCHECK(hipStreamSynchronize(c->ex->stream));
-    std::fill(c->host_valid.begin(), c->host_valid.end(), 0);
-    std::fill(c->ticked_valid.begin(), c->ticked_valid.end(), 0);
+    for (auto &f : c->host_valid) f = 0;
     for (int b : rows) c->ticked_valid[b] = 1;
-    std::fill(c->wanted.begin(), c->wanted.end(), 0);
+    for (auto &f : c->wanted) f = 0;
     c->tick++;
 }
 
 const void *stream_current(StreamCtx *c, size_t handle) {
     if (handle >= (size_t)c->m->nbuf) throw Error("bad buffer handle");
     c->wanted[handle] = 1;
-    if (!c->host_valid[handle] && c->ticked_valid[handle]) {
+    if (c->host_valid[handle]) return c->host_rows[handle];
+    std::lock_guard<std::mutex> g(c->ex->mu); // a tick that runs ends first
+    if (c->host_valid[handle]) return c->host_rows[handle];
+    if (c->ticked_valid[handle]) {
         memcpy(c->host_rows[handle], c->ticked[handle], c->esz * c->S);
-        c->host_valid[handle] = 1;
-    }
-    if (!c->host_valid[handle]) {
-        std::lock_guard<std::mutex> g(c->ex->mu);
+    } else {
         HIPCHECK(hipMemcpyAsync(c->host_rows[handle], c->rows[handle], c->esz * c->S, hipMemcpyDeviceToHost,
                                 c->ex->stream));
         HIPCHECK(hipStreamSynchronize(c->ex->stream));
-        c->host_valid[handle] = 1;
     }
+    c->host_valid[handle] = 1;
     return c->host_rows[handle];
 }
 
 const void *stream_current_device(StreamCtx *c, size_t handle) {
     if (handle >= (size_t)c->m->nbuf) throw Error("bad buffer handle");
+    if (c->exposed[handle]) return c->rows[handle];
+    std::lock_guard<std::mutex> g(c->ex->mu);
     c->exposed[handle] = 1;
     c->ticked_valid[handle] = 0; // the caller may write the row now
     return c->rows[handle];

@@ -610,7 +610,13 @@ void plan_nodes(const KunModuleDesc *m, size_t S, size_t L, int lanes, BatchLayo
     // would save no more than their cost, one lane takes every kernel (4
     // kernels of 64 x 260: 46 us against 79; Rank and Scale of two inputs
     // over 1024 rows of 8192 floats: 128 us against 153, over 750 rows of
-    // 5003 doubles 143 against 163).
+    // 5003 doubles 143 against 163). The same plan holds for each job of a
+    // batch: enqueued, one of the first takes 49 us against 120 with lanes
+    // and two 106 against 165; as a graph, where a branch is not free either,
+    // two take 87 us against 147, six of Rank and Scale over 250 rows of 500
+    // floats 155 against 740. Only one long job as a graph is better with
+    // lanes (1024 rows of 8192 floats: 146 us against 159, alone 190 against
+    // 174).
     if (sum - std::max(span, full) < 30.0)
         for (auto &nd : lay.nodes) nd.lane = 0;
 }
@@ -626,6 +632,31 @@ void enqueue_batch_serial(const KunModuleDesc *m, const std::vector<void *> &dev
     if (L == 0) return;
     for (const auto &nd : lay.nodes) enqueue_node(m, nd.stage, nd.kern, dev, lay, arena, S, T, start, L, st, prof);
 }
+
+// The lanes that a set of nodes uses, forked from `st` and joined into it; a
+// single lane is `st` itself, with no events at all.
+struct LaneFork {
+    Executor &ex;
+    hipStream_t st;
+    std::vector<char> used;
+    bool alone;
+    LaneFork(Executor &ex_, const std::vector<int> &lane, hipStream_t st_) : ex(ex_), st(st_), used(ex_.lanes.size(), 0) {
+        for (int l : lane) used[l] = 1;
+        alone = std::count(used.begin(), used.end(), 1) <= 1;
+        if (alone) return;
+        HIPCHECK(hipEventRecord(ex.fork, st));
+        for (size_t l = 0; l < used.size(); l++)
+            if (used[l]) HIPCHECK(hipStreamWaitEvent(ex.lanes[l], ex.fork, 0));
+    }
+    hipStream_t stream(int l) const { return alone ? st : ex.lanes[l]; }
+    void join() const {
+        for (size_t l = 0; l < used.size(); l++) {
+            if (alone || !used[l]) continue;
+            HIPCHECK(hipEventRecord(ex.lane_done[l], ex.lanes[l]));
+            HIPCHECK(hipStreamWaitEvent(st, ex.lane_done[l], 0));
+        }
+    }
+};
 
 void enqueue_batch(Executor &ex, const KunModuleDesc *m, const std::vector<void *> &dev, const BatchLayout &lay,
                    char *arena, size_t S, size_t T, size_t start, size_t L, hipStream_t st) {
@@ -648,26 +679,17 @@ void enqueue_batch(Executor &ex, const KunModuleDesc *m, const std::vector<void 
         w.sync_lanes = nl;
     }
     ex.ensure_stage_events((int)lay.nodes.size());
-    std::vector<char> used(nl, 0);
-    for (const auto &nd : lay.nodes) used[nd.lane % nl] = 1;
-    const bool alone = std::count(used.begin(), used.end(), 1) <= 1;
-    if (!alone) {
-        HIPCHECK(hipEventRecord(ex.fork, st));
-        for (int l = 0; l < nl; l++)
-            if (used[l]) HIPCHECK(hipStreamWaitEvent(ex.lanes[l], ex.fork, 0));
-    }
+    std::vector<int> lane;
+    for (const auto &nd : lay.nodes) lane.push_back(nd.lane % nl);
+    const LaneFork fork(ex, lane, st);
     for (size_t n = 0; n < lay.nodes.size(); n++) {
         const auto &nd = lay.nodes[n];
-        hipStream_t ls = alone ? st : ex.lanes[nd.lane % nl];
+        hipStream_t ls = fork.stream(lane[n]);
         for (int d : lay.sync.waits[n]) HIPCHECK(hipStreamWaitEvent(ls, ex.stage_done[d], 0));
         enqueue_node(m, nd.stage, nd.kern, dev, lay, arena, S, T, start, L, ls, prof);
         if (lay.sync.record[n]) HIPCHECK(hipEventRecord(ex.stage_done[n], ls));
     }
-    for (int l = 0; l < nl; l++) {
-        if (alone || !used[l]) continue;
-        HIPCHECK(hipEventRecord(ex.lane_done[l], ex.lanes[l]));
-        HIPCHECK(hipStreamWaitEvent(st, ex.lane_done[l], 0));
-    }
+    fork.join();
 }
 
 void check_batch_module(const KunModuleDesc *m, size_t S, size_t T, size_t start, size_t L) {
@@ -847,8 +869,6 @@ static void enqueue_jobs(Executor &ex, const std::vector<BatchJob> &jobs, const 
         return;
     }
     ex.ensure_stage_events((int)first.back());
-    HIPCHECK(hipEventRecord(ex.fork, st));
-    for (int l = 0; l < nl; l++) HIPCHECK(hipStreamWaitEvent(ex.lanes[l], ex.fork, 0));
     // enqueue order: one node of each job in turn (job j shifted j lanes),
     // items numbered in that order; events are indexed by job and node
     std::vector<std::pair<size_t, size_t>> order; // (job, node)
@@ -871,20 +891,20 @@ static void enqueue_jobs(Executor &ex, const std::vector<BatchJob> &jobs, const 
         for (int d : nd.deps) deps[i].push_back(item_of[first[j] + d]);
     }
     const LaneSync sync = plan_lane_sync(lane, deps, nl);
+    // only lanes in use fork and join; one lane is `st` itself, as in
+    // enqueue_batch
+    const LaneFork fork(ex, lane, st);
     for (size_t i = 0; i < order.size(); i++) {
         const size_t j = order[i].first, n = order[i].second;
         const auto &nd = temps[j]->lay.nodes[n];
-        hipStream_t ls = ex.lanes[lane[i]];
+        hipStream_t ls = fork.stream(lane[i]);
         for (int d : sync.waits[i])
             HIPCHECK(hipStreamWaitEvent(ls, ex.stage_done[first[order[d].first] + order[d].second], 0));
         enqueue_node(jobs[j].m, nd.stage, nd.kern, dev[j], temps[j]->lay, temps[j]->arena, jobs[j].S, jobs[j].T,
                      jobs[j].start, jobs[j].L, ls, prof);
         if (sync.record[i]) HIPCHECK(hipEventRecord(ex.stage_done[first[j] + n], ls));
     }
-    for (int l = 0; l < nl; l++) {
-        HIPCHECK(hipEventRecord(ex.lane_done[l], ex.lanes[l]));
-        HIPCHECK(hipStreamWaitEvent(st, ex.lane_done[l], 0));
-    }
+    fork.join();
 }
 
 static void check_jobs(const std::vector<BatchJob> &jobs) {

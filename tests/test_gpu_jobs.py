@@ -128,3 +128,29 @@ def test_autotune_keeps_results(batch):
     bad = [k for k in got if not _same(got[k], alone[j][k])]
     assert not bad, f"tuned chunking {best} changed outputs {bad[:3]}"
 
+
+
+@pytest.mark.parametrize("name,S,T", [("simple_f32", 64, 260), ("cs_f32", 500, 250), ("jobs_g0", 100, 250)])
+@pytest.mark.parametrize("count", [1, 2])
+def test_few_jobs_on_a_callers_stream(name, S, T, count):
+    """Batches that use one lane (the caller's stream itself) or a few: the
+    caller's writes before, and reads after, need no other order."""
+    _, mod = catalog.load(name)
+    ex = kr.createSingleThreadExecutor()
+    d = data.ohlcv(S, T, seed=S, nan_frac=0.1)
+    ins = {k: d.get(k, d["close"]) for k in mod.getInputNames()}
+    exp = kr.runGraph(ex, mod, ins, 0, T)
+    host = {k: torch.from_numpy(v).pin_memory() for k, v in ins.items()}
+    st = torch.cuda.Stream()
+    with torch.cuda.stream(st):
+        for rep in range(3):
+            dev = [{k: torch.empty((T, S), device="cuda") for k in ins} for _ in range(count)]
+            out = [{k: torch.full((T, S), 12345.0, device="cuda") for k in exp} for _ in range(count)]
+            for j in dev:
+                for k, v in j.items():
+                    v.copy_(host[k], non_blocking=True)
+            kr.runGraphBatchDevice(ex, [(mod, {k: v.data_ptr() for k, v in {**i, **o}.items()}, S, T, 0, T)
+                                        for i, o in zip(dev, out)], stream=st.cuda_stream)
+            got = [{k: v.cpu().numpy() for k, v in o.items()} for o in out]
+            for g in got:
+                assert not [k for k in exp if not _same(g[k], exp[k])], rep

@@ -565,9 +565,13 @@ void plan_nodes(const KunModuleDesc *m, size_t S, size_t L, int lanes, BatchLayo
                 for (int j = 0; j < sd.nin; j++)
                     if (writer[sd.in[j]] >= 0) nd.deps.push_back(writer[sd.in[j]]);
                 for (int j = 0; j < sd.nout; j++) writer[sd.out[j]] = id;
-                // 37 / 27 us for 1024 rows of 8192 floats; doubles twice that
-                nd.est = 8.0 + (double)L * (sd.kind == KUN_STAGE_RANK ? 0.03 : 0.02) * (double)S / 8192.0 *
-                                   (elem_size(m) == 8 ? 2.0 : 1.0);
+                // a generic op's lane walks its row, 0.43 us a stock for
+                // 300 rows as for 1024; Rank and Scale: 37 / 27 us for 1024
+                // rows of 8192 floats, doubles twice that
+                nd.est = sd.kind == KUN_STAGE_GENERIC
+                             ? 8.0 + 0.43 * (double)S
+                             : 8.0 + (double)L * (sd.kind == KUN_STAGE_RANK ? 0.03 : 0.02) * (double)S / 8192.0 *
+                                         (elem_size(m) == 8 ? 2.0 : 1.0);
             }
             std::sort(nd.deps.begin(), nd.deps.end());
             nd.deps.erase(std::unique(nd.deps.begin(), nd.deps.end()), nd.deps.end());
@@ -601,8 +605,10 @@ void plan_nodes(const KunModuleDesc *m, size_t S, size_t L, int lanes, BatchLayo
         finish[n] = best_start + nd.est;
         lane_free[best] = finish[n];
         sum += nd.est;
-        // a workgroup a row: 256 rows occupy every CU
-        if (m->stages[nd.stage].kind != KUN_STAGE_TS && L >= 256) full += nd.est;
+        // Rank and Scale have a workgroup a row: 256 rows occupy every CU
+        // (a generic op has a lane a row)
+        const int kind = m->stages[nd.stage].kind;
+        if ((kind == KUN_STAGE_RANK || kind == KUN_STAGE_SCALE) && L >= 256) full += nd.est;
         span = std::max(span, finish[n]);
     }
     // The fork, the events and the join of the lanes cost about 35 us, and

@@ -6,7 +6,7 @@ import os
 from typing import Callable, Dict, Tuple
 
 from .. import PACKAGE_DIR
-from .graphs import (aligned_graph, alpha101_graph, large_window_graph, capi_batch_graph, capi_stream_graph, alpha158_graph, cross_section_graph, generic_cs_graph, generic_pair_graph, tsrank_chain_graph, ops_graph, precision_graph, random_graph, simple_graph,
+from .graphs import (aligned_graph, alpha101_graph, large_window_graph, capi_batch_graph, capi_stream_graph, alpha158_graph, cross_section_graph, generic_cs_graph, generic_pair_graph, generic_two_graph, tsrank_chain_graph, ops_graph, precision_graph, random_graph, simple_graph,
                      stream_graph)
 
 MODULE_DIR = os.path.join(PACKAGE_DIR, "lib", "modules")
@@ -53,6 +53,7 @@ CATALOG: Dict[str, Tuple[Callable, dict]] = {
                                                options={"no_fast_stat": "no_warn"})),
     "generic_stream_f32": (generic_cs_graph, dict(input_layout="STREAM", output_layout="STREAM")),
     "generic_pair_f32": (generic_pair_graph, dict(input_layout="TS", output_layout="TS")),
+    "generic_two_f32": (generic_two_graph, dict(input_layout="TS", output_layout="TS")),
     # graphs of the batched-jobs workload (64 uneven jobs draw from this pool)
     "jobs_g0": (lambda: random_graph(20, 4000), dict(input_layout="TS", output_layout="TS")),
     "jobs_g1": (lambda: random_graph(30, 4001), dict(input_layout="TS", output_layout="TS")),

@@ -385,6 +385,17 @@ def generic_pair_graph(K=None):
     return K.Function(b.ops)
 
 
+def generic_two_graph(K=None):
+    """Two generic cross-sectional ops straight off the inputs."""
+    K = K or native()
+    b = K.Builder()
+    with b:
+        a, c = K.Input("a"), K.Input("c")
+        K.Output(K.DiffWithWeightedSum(a, c), "a_c")
+        K.Output(K.DiffWithWeightedSum(c, a), "c_a")
+    return K.Function(b.ops)
+
+
 def cross_section_graph(K=None):
     """Rank and Scale straight off the inputs (cross-sectional kernel checks)."""
     K = K or native()

@@ -136,6 +136,10 @@ def test_module_cache_key_changes_with_each_load():
     ("cs_f64", 16384, 200, False),     # the same with long rows: lanes pay
     ("ops_f32", 200, 100, False),
     ("cfg2_f32", 8192, 1024, False),
+    # generic ops: a lane a row, which fills nothing however many rows
+    ("generic_two_f32", 8, 300, True),
+    ("generic_two_f32", 500, 300, False),
+    ("generic_two_f32", 8192, 1024, False),
 ])
 def test_runs_keep_to_one_lane_where_lanes_save_nothing(name, stocks, days, one):
     _, mod = catalog.load(name)

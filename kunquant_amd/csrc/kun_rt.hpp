@@ -59,7 +59,19 @@ struct Pool {
     std::multimap<size_t, void *> free_;
     void *get(size_t bytes);
     void put(void *p, size_t bytes);
+    void trim(); // frees what is cached
     ~Pool();
+};
+
+// One piece of device memory that grows to the largest size asked for
+struct Workspace {
+    char *p = nullptr;
+    size_t bytes = 0;
+    // at least n bytes (what an earlier call left there is lost), or false
+    // where the device has not that much left; nothing may be using it
+    bool reserve(size_t n, Pool &pool);
+    void free();
+    ~Workspace() { free(); }
 };
 
 // Device memory of a batch run, one arena: per kernel, its row chunking and
@@ -130,6 +142,7 @@ struct Executor {
     hipEvent_t fork = nullptr;
     void ensure_stage_events(int n);
     Pool pool;
+    Workspace corr; // copies and ranks of corrWith's inputs
     std::mutex mu;
     ChunkPolicy chunking;
     // temporaries of device-resident runs, per (module, load serial, stocks,

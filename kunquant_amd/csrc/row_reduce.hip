@@ -275,26 +275,38 @@ void corr_with(Executor &ex, bool device, int sts, bool rank_inputs, int n, cons
     HIPCHECK(hipSetDevice(ex.device));
     if (!st) st = ex.stream;
     const size_t in_bytes = (sts ? (S + blk - 1) / blk * blk : S) * T * sizeof(float);
-    // a launch takes a group of inputs: as many as it can, and device copies
-    // and ranks together within a gigabyte
-    const size_t out_bytes = L * sizeof(float) + 4, rank_bytes = S * L * sizeof(float) + 4;
-    const size_t each = (device ? 0 : in_bytes + out_bytes) + (rank_inputs ? rank_bytes : 0);
-    const size_t fit = each ? std::max<size_t>(1, ((size_t)1 << 30) / each) : (size_t)kun_cs::corr_inputs();
-    const int group = (int)std::min<size_t>(std::min<size_t>(fit, (size_t)kun_cs::corr_inputs()), (size_t)n);
-    std::unique_ptr<DevBuf> dtarget;
-    std::vector<std::unique_ptr<DevBuf>> dx, dout, ranks;
-    const float *y = target;
-    if (!device) {
-        dtarget.reset(new DevBuf(ex, in_bytes));
-        HIPCHECK(hipMemcpyAsync(dtarget->p, target, in_bytes, hipMemcpyHostToDevice, st));
-        y = (const float *)dtarget->p;
-    }
-    for (int k = 0; k < group; k++) {
-        if (!device) {
-            dx.emplace_back(new DevBuf(ex, in_bytes));
-            dout.emplace_back(new DevBuf(ex, out_bytes));
+    // a launch takes a group of inputs: as many as it can, device copies and
+    // ranks together within a gigabyte, or fewer where the device has less
+    auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
+    const size_t x_bytes = device ? 0 : up(in_bytes), o_bytes = device ? 0 : up(L * sizeof(float) + 4);
+    const size_t r_bytes = rank_inputs ? up(S * L * sizeof(float) + 4) : 0;
+    const size_t each = x_bytes + o_bytes + r_bytes, most = (size_t)1 << 30;
+    size_t fit = (size_t)kun_cs::corr_inputs();
+    if (each) fit = std::min(fit, std::max<size_t>(1, most > x_bytes ? (most - x_bytes) / each : 0));
+    int group = (int)std::min<size_t>(fit, (size_t)n);
+    while (group > 1 && each && !ex.corr.reserve(x_bytes + group * each, ex.pool)) group /= 2;
+    if (group && each && !ex.corr.reserve(x_bytes + group * each, ex.pool))
+        throw Error("hipMalloc of " + std::to_string(x_bytes + group * each) + " bytes for corrWith failed");
+    // the workspace is free again when the call returns, also by an error
+    struct Wait {
+        hipStream_t st;
+        bool on;
+        ~Wait() {
+            if (on) hipStreamSynchronize(st);
         }
-        if (rank_inputs) ranks.emplace_back(new DevBuf(ex, rank_bytes));
+    } wait{st, each != 0};
+    const float *y = target;
+    char *at = ex.corr.p;
+    if (!device && n) {
+        HIPCHECK(hipMemcpyAsync(at, target, in_bytes, hipMemcpyHostToDevice, st));
+        y = (const float *)at;
+        at += x_bytes;
+    }
+    std::vector<char *> dx, dout, ranks;
+    for (int k = 0; k < group; k++, at += each) {
+        dx.push_back(at);
+        dout.push_back(at + x_bytes);
+        ranks.push_back(at + x_bytes + o_bytes);
     }
     for (int i0 = 0; i0 < n; i0 += group) {
         const int m = std::min(group, n - i0);
@@ -305,14 +317,14 @@ void corr_with(Executor &ex, bool device, int sts, bool rank_inputs, int n, cons
             x[k] = inputs[i0 + k];
             o[k] = outs[i0 + k];
             if (!device) {
-                HIPCHECK(hipMemcpyAsync(dx[k]->p, x[k], in_bytes, hipMemcpyHostToDevice, st));
-                x[k] = (const float *)dx[k]->p;
-                o[k] = (float *)dout[k]->p;
+                HIPCHECK(hipMemcpyAsync(dx[k], x[k], in_bytes, hipMemcpyHostToDevice, st));
+                x[k] = (const float *)dx[k];
+                o[k] = (float *)dout[k];
             }
             if (rank_inputs && e == hipSuccess) {
-                kun_cs::View vi{(void *)x[k], sts ? 0 : 1, (long)T, (long)start}, vo{ranks[k]->p, 1, (long)L, 0};
+                kun_cs::View vi{(void *)x[k], sts ? 0 : 1, (long)T, (long)start}, vo{ranks[k], 1, (long)L, 0};
                 e = kun_cs::launch_rank(0, vi, vo, (long)S, (long)L, blk, st);
-                x[k] = (const float *)ranks[k]->p;
+                x[k] = (const float *)ranks[k];
             }
         }
         if (e == hipSuccess)
@@ -325,8 +337,8 @@ void corr_with(Executor &ex, bool device, int sts, bool rank_inputs, int n, cons
             for (int k = 0; k < m; k++)
                 HIPCHECK(hipMemcpyAsync(outs[i0 + k], o[k], L * sizeof(float), hipMemcpyDeviceToHost, st));
     }
-    // host buffers are copied back; pooled scratch returns to the pool only
-    // once the kernels reading it are done
+    // host buffers are copied back, the workspace is free
+    wait.on = false;
     if (!device || rank_inputs) HIPCHECK(hipStreamSynchronize(st));
 }
 

@@ -71,8 +71,35 @@ void Pool::put(void *p, size_t bytes) {
     free_.emplace(bytes, p);
 }
 
-Pool::~Pool() {
+void Pool::trim() {
+    std::lock_guard<std::mutex> g(mu);
     for (auto &kv : free_) hipFree(kv.second);
+    free_.clear();
+}
+
+Pool::~Pool() { trim(); }
+
+bool Workspace::reserve(size_t n, Pool &pool) {
+    if (n <= bytes) return true;
+    free();
+    hipError_t e = hipMalloc((void **)&p, n);
+    if (e != hipSuccess) {
+        pool.trim();
+        e = hipMalloc((void **)&p, n);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        p = nullptr;
+        return false;
+    }
+    bytes = n;
+    return true;
+}
+
+void Workspace::free() {
+    if (p) hipFree(p);
+    p = nullptr;
+    bytes = 0;
 }
 
 Executor::Executor() : chunking(ChunkPolicy::from_env()) {
@@ -1164,6 +1191,7 @@ std::string describe_jobs_graph(const std::vector<BatchJob> &jobs, int lanes) {
 void Executor::free_temps() {
     for (auto &kv : temps) free_device_temps(kv.second);
     temps.clear();
+    corr.free();
 }
 
 } // namespace kunrt

@@ -1,15 +1,11 @@
 // Rows read by one thread while another runs ticks: every row returned is one
-// tick's. The HIP calls of libkunhip.so are answered here by host memory (this
-// program's symbols come before the HIP runtime's), so that a tick's parts can
-// be slowed down: a launch of the tick's kernels sets every output row to the
+// tick's. The HIP calls of libkunhip.so are answered by host memory, so that a
+// tick's parts can be slowed down: a launch of the tick's kernels sets every output row to the
 // tick's number; the launch that copies rows to the host, and the reader's own
 // copies of a row, take it in two halves with a pause between them.
 // Arguments: module name, its library. Exits 1 on a row of two ticks or one
 // older than the last tick that had ended before the read began.
-#include <dlfcn.h>
 #include <stdio.h>
-#include <stdlib.h>
-#include <string.h>
 #include <unistd.h>
 
 #include <atomic>
@@ -18,10 +14,8 @@
 #include <vector>
 
 #include "../../include/kun_capi.h"
+#include "host_hip.hpp"
 #include "kun_module_abi.h"
-
-typedef void *P;
-struct Dim { unsigned x, y, z; };
 
 static const size_t S = 512;
 static std::mutex alloc_mu;
@@ -40,43 +34,16 @@ extern "C" __attribute__((visibility("default"))) void *memcpy(void *d, const vo
     return d;
 }
 
-#define FAKE extern "C" __attribute__((visibility("default"))) int
-FAKE hipMalloc(P *p, size_t n) {
-    *p = calloc(1, n + 1);
+P host_alloc(size_t n) {
+    P p = calloc(1, n + 1);
     std::lock_guard<std::mutex> g(alloc_mu);
-    if (n == S * sizeof(double)) device_rows.push_back(*p);
-    return 0;
+    if (n == S * sizeof(double)) device_rows.push_back(p);
+    return p;
 }
-FAKE hipFree(P p) { free(p); return 0; }
-FAKE hipHostMalloc(P *p, size_t n, unsigned) { *p = calloc(1, n + 1); return 0; }
-FAKE hipHostFree(P p) { free(p); return 0; }
-FAKE hipMemcpy(P d, const void *s, size_t n, int) { memcpy(d, s, n); return 0; }
-FAKE hipMemcpyAsync(P d, const void *s, size_t n, int, P) { memcpy(d, s, n); return 0; }
-FAKE hipSetDevice(int) { return 0; }
-FAKE hipGetDevice(int *d) { *d = 0; return 0; }
-FAKE hipGetLastError() { return 0; }
-FAKE hipDeviceSynchronize() { return 0; }
-FAKE hipStreamCreateWithFlags(P *s, unsigned) { *s = malloc(1); return 0; }
-FAKE hipStreamDestroy(P s) { free(s); return 0; }
-FAKE hipStreamSynchronize(P) { return 0; }
-FAKE hipStreamWaitEvent(P, P, unsigned) { return 0; }
-FAKE hipEventCreate(P *e) { *e = malloc(1); return 0; }
-FAKE hipEventCreateWithFlags(P *e, unsigned) { *e = malloc(1); return 0; }
-FAKE hipEventDestroy(P e) { free(e); return 0; }
-FAKE hipEventRecord(P, P) { return 0; }
-FAKE hipEventSynchronize(P) { return 0; }
+void host_free(P p) { free(p); }
 
-static thread_local struct { Dim g, b; size_t sh; P st; } config;
-extern "C" __attribute__((visibility("default"))) int __hipPushCallConfiguration(Dim g, Dim b, size_t sh, P st) {
-    config = {g, b, sh, st};
-    return 0;
-}
-extern "C" __attribute__((visibility("default"))) int __hipPopCallConfiguration(Dim *g, Dim *b, size_t *sh, P *st) {
-    *g = config.g, *b = config.b, *sh = config.sh, *st = config.st;
-    return 0;
-}
 static const void *copy_kernel = nullptr; // the one launched for several rows at once
-FAKE hipLaunchKernel(const void *func, Dim grid, Dim, P *args, size_t, P) {
+int host_launch(const void *func, Dim grid, Dim, P *args) {
     if (grid.y >= 2) copy_kernel = func;
     if (func == copy_kernel) { // rows to the host: {sources[64], destinations[64]}
         P *rows = (P *)args[0];

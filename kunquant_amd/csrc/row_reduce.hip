@@ -192,23 +192,27 @@ hipError_t launch_corr(int n, const float *const *x, int xsts, long xT, long xro
                        float *const *out, long S, long start, long L, int blk, hipStream_t st) {
     if (L <= 0 || n <= 0) return hipSuccess;
     if (n > CORR_INPUTS) return hipErrorInvalidValue;
-    CorrArgs a;
-    for (int i = 0; i < CORR_INPUTS; i++) {
-        a.x[i] = x[i < n ? i : 0];
-        a.out[i] = out[i < n ? i : 0];
+    // a grid has fewer than 2^32 threads
+    const long per = 1L << 24;
+    for (long l0 = 0; l0 < L; l0 += per) {
+        CorrArgs a;
+        for (int i = 0; i < CORR_INPUTS; i++) {
+            a.x[i] = x[i < n ? i : 0];
+            a.out[i] = out[i < n ? i : 0] + l0;
+        }
+        a.y = y;
+        a.xsts = xsts;
+        a.ysts = ysts;
+        a.blk = blk;
+        a.xT = xT;
+        a.xrow0 = xrow0 + l0;
+        a.yT = yT;
+        a.S = S;
+        a.start = start + l0;
+        a.L = L - l0 < per ? L - l0 : per;
+        hipLaunchKernelGGL(corr_rows, dim3((unsigned)((a.L + CORR_ROWS - 1) / CORR_ROWS), (unsigned)n),
+                           dim3(CORR_BLOCK), 0, st, a);
     }
-    a.y = y;
-    a.xsts = xsts;
-    a.ysts = ysts;
-    a.blk = blk;
-    a.xT = xT;
-    a.xrow0 = xrow0;
-    a.yT = yT;
-    a.S = S;
-    a.start = start;
-    a.L = L;
-    hipLaunchKernelGGL(corr_rows, dim3((unsigned)((L + CORR_ROWS - 1) / CORR_ROWS), (unsigned)n), dim3(CORR_BLOCK), 0,
-                       st, a);
     return hipGetLastError();
 }
 

@@ -2,8 +2,8 @@
 // smaller groups; over calls of many shapes, what the executor keeps is
 // bounded. The HIP calls of libkunhip.so are answered by host memory (kernels
 // do nothing); the launches say how many rows of how many inputs were ranked
-// and summed. Exits 1 where a call fails, an input is left out or too much is
-// kept.
+// and summed. Exits 1 where a call fails, an input or row is left out, a launch
+// has more threads than a grid may have or too much is kept.
 #include <stdio.h>
 
 #include <map>
@@ -14,7 +14,7 @@
 
 static std::map<P, size_t> live;
 static size_t held = 0, limit = ~(size_t)0;
-static long ranked = 0, summed = 0;
+static long ranked = 0, summed = 0, groups = 0, wide = 0;
 
 P host_alloc(size_t n) {
     if (held + n > limit) return nullptr;
@@ -30,8 +30,13 @@ void host_free(P p) {
     free(p);
 }
 int host_launch(const void *, Dim grid, Dim block, P *) {
-    if (block.x == 320) summed += grid.y; // the sums: a wavefront of chains and four that load
-    else ranked += grid.x;
+    if ((size_t)grid.x * block.x >> 32) wide++;
+    if (block.x == 320) { // the sums: a wavefront of chains and four that load
+        summed += grid.y;
+        groups += (long)grid.x * grid.y;
+    } else {
+        ranked += grid.x;
+    }
     return 0;
 }
 
@@ -66,6 +71,13 @@ int main() {
     call(8000, 20000, "panels of 640 MB");
     if (held > (size_t)1 << 30) {
         printf("%zu bytes kept\n", held);
+        bad++;
+    }
+    groups = 0; // of 8 rows
+    const size_t rows = (size_t)1 << 28;
+    if (kunCorrWithDevice(ex, 1, 0, 3, x.data(), y, o.data(), 1, rows + 5, 0, rows + 5, nullptr) || wide ||
+        groups != 3 * (long)(rows / 8 + 1)) {
+        printf("2^28 rows: %ld groups, %ld launches too wide\n", groups, wide);
         bad++;
     }
     kunDestoryExecutor(ex);

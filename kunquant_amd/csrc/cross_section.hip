@@ -686,8 +686,12 @@ template <typename T, int BLOCK, int ITEMS> struct CountRank {
 // Buckets of more than DEEP keys are whole tie groups as a rule (discrete
 // values): a lane whose key differs from its bucket's first one raises a
 // flag, and unless some bucket of the row is both deep and mixed, a deep
-// bucket's bounds are the tie group's. Returns false, with nothing written,
-// if the row has such a bucket; the caller then sorts it.
+// bucket's bounds are the tie group's. A row with such a bucket (values close
+// together beside distant ones) is cut once more:
+//  6. every bucket's range is divided evenly by two positions for each of its
+//     keys, as coarse buckets were, and 3. to 5. follow.
+// Where a bucket is deep and mixed after that too (clusters within clusters),
+// nothing has been written and the row is sorted.
 //
 // 2 N positions (FSH = 0), or N / 2 (FSH = 2) where 64-bit keys leave less
 // LDS.
@@ -695,7 +699,11 @@ template <typename T, int BLOCK, int ITEMS> struct CountRank {
 // 1024 rows of 8192 floats: 37 us a launch, 92 by the sort (floor 13 us at
 // the card's copy rate); 750 rows of 5003 doubles: 43 against 191, the sort
 // needing 16 passes; one row of 5000 doubles: 12 against 54; a pool cycle's
-// Rank segments of about 2200 stocks: 7.9 against 15. Bound by LDS accesses
+// Rank segments of about 2200 stocks: 7.9 against 15. Rows of values within
+// 1e-4 of each other and one of 1e30: 97 us for 1024 of 8192 floats (142 when
+// such rows were sorted after the first cut, 92 by the sort alone), 69 for 750
+// of 5003 doubles (227, 191). Within 1e-9, doubles end in the sort: 273 us, 246
+// after one cut. Bound by LDS accesses
 // and the instructions around them (about ten accesses a key, most of them
 // to random banks). Two workgroups a CU are worth 43 -> 37 us for float rows
 // of 8192 and take 64 registers, so values are packed and taken apart again
@@ -716,7 +724,9 @@ template <typename T, int BLOCK, int ITEMS, int FSH> struct BucketRank {
         uint32_t coarse[NC + 1];   // counts, then first keys
         K wmax[NW], wmin[NW];
         uint32_t wn[NW], wc[NW], wf[NW];
-        uint32_t mixed;
+        uint32_t mixed[2], n;
+        int sh;
+        K kmin;
     };
 
     static __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
@@ -742,7 +752,8 @@ template <typename T, int BLOCK, int ITEMS, int FSH> struct BucketRank {
         return w ? lane_value(p, w - 1) : 0u;
     }
 
-    template <int LIN, int LOUT>
+    // AGAIN: the row that this function left before with deep mixed buckets
+    template <int LIN, int LOUT, bool AGAIN>
     static __device__ __forceinline__ bool row(Smem &sm, const kun_cs::View &in, const kun_cs::View &out, long S,
                                                int blk, long t) {
         const int tid = threadIdx.x, lane = tid & 63;
@@ -751,91 +762,124 @@ template <typename T, int BLOCK, int ITEMS, int FSH> struct BucketRank {
         T *dst = (T *)out.ptr;
         const long rin = t + in.row0;
         const int n_all = (int)S;
-        T xs[ITEMS];
-#pragma unroll
-        for (int j = 0; j < ITEMS; j++) {
-            const int left = n_all - j * BLOCK;
-            if (left > 0) xs[j] = *cell_at<LIN>(src, in, rin, j * BLOCK, min(tid, left - 1), S, blk);
-        }
-#pragma unroll
-        for (int i = 0; i < CW; i++) sm.coarse[i * BLOCK + tid] = 0;
-#pragma unroll
-        for (int i = 0; i < FW; i++) sm.fine[i * BLOCK + tid] = 0;
-        if (tid == 0) sm.mixed = 0;
         K key[ITEMS]; // ~0: missing
-        K kmax = 0, kinv = 0;
+        K kmin;
         uint32_t n = 0;
-#pragma unroll
-        for (int j = 0; j < ITEMS; j++) {
-            key[j] = tid < n_all - j * BLOCK ? rank_key(xs[j]) : ~K(0);
-            const bool live = key[j] != ~K(0);
-            n += (uint32_t)__popcll(__ballot(live));
-            const K a = live ? key[j] : K(0), b = ~key[j];
-            kmax = a > kmax ? a : kmax;
-            kinv = b > kinv ? b : kinv; // a missing cell's is 0
-        }
-        kmax = wave_max(kmax);
-        kinv = wave_max(kinv);
-        if (lane == 0) {
-            sm.wmax[w] = kmax;
-            sm.wmin[w] = kinv;
-            sm.wn[w] = n;
-        }
-        __syncthreads();
-        // lane q < NW holds wavefront q's
-        n = lane_value(dpp_row_incl_sum(lane < NW ? sm.wn[lane] : 0u), NW - 1);
-        kmax = wave_max(lane < NW ? sm.wmax[lane] : K(0));
-        kinv = wave_max(lane < NW ? sm.wmin[lane] : K(0));
-        const K kmin = ~kinv;
-        int sh = 0; // bits of key - kmin below the coarse bucket's
-        if (n && kmax != kmin) {
-            const K range = kmax - kmin;
-            const int bits = sizeof(K) == 8 ? 64 - __builtin_clzll((uint64_t)range) : 32 - __builtin_clz((uint32_t)range);
-            constexpr int CB = __builtin_ctz(NC);
-            sh = bits > CB ? bits - CB : 0;
-        }
-        sh = __builtin_amdgcn_readfirstlane(sh);
-        // Missing cells go through the same instructions, adding nothing to a
-        // count of their lane's own and storing the largest pattern where the
-        // keys end with it anyway: no branch per cell.
-        // 1. coarse counts
-#pragma unroll
-        for (int j = 0; j < ITEMS; j++) {
-            const bool live = key[j] != ~K(0);
-            atomicAdd(&sm.coarse[live ? (uint32_t)((key[j] - kmin) >> sh) : (uint32_t)tid], live ? 1u : 0u);
-        }
-        __syncthreads();
-        // 2. first keys of the coarse buckets
-        {
-            uint32_t c[CW], s = 0;
-#pragma unroll
-            for (int i = 0; i < CW; i++) {
-                c[i] = sm.coarse[tid * CW + i];
-                s += c[i];
-            }
-            const uint32_t incl = dpp_incl_sum(s);
-            if (lane == 63) sm.wc[w] = incl;
-            __syncthreads();
-            uint32_t run = before(sm.wc, w, lane) + incl - s;
-#pragma unroll
-            for (int i = 0; i < CW; i++) {
-                sm.coarse[tid * CW + i] = run;
-                run += c[i];
-            }
-            if (tid == 0) sm.coarse[NC] = n;
-        }
-        __syncthreads();
-        // 3. positions, and each key's turn in its bucket
+        int sh = 0;         // bits of key - kmin below the coarse bucket's
         uint32_t at[ITEMS]; // position, turn in the high half
+        if constexpr (!AGAIN) {
+            T xs[ITEMS];
 #pragma unroll
-        for (int j = 0; j < ITEMS; j++) {
-            const K r = key[j] != ~K(0) ? key[j] - kmin : K(0);
-            const uint32_t b = (uint32_t)(r >> sh);
-            const uint32_t c0 = sm.coarse[b], c1 = sm.coarse[b + 1];
-            // the bits below the bucket's, as a 32-bit fraction of its range
-            constexpr int TOP = (int)sizeof(K) * 8 - 1;
-            const uint32_t frac = (uint32_t)(((r << 1) << (TOP - sh)) >> (TOP - 31));
-            at[j] = (2 * c0 + __umulhi(frac, 2 * (c1 - c0))) >> FSH;
+            for (int j = 0; j < ITEMS; j++) {
+                const int left = n_all - j * BLOCK;
+                if (left > 0) xs[j] = *cell_at<LIN>(src, in, rin, j * BLOCK, min(tid, left - 1), S, blk);
+            }
+#pragma unroll
+            for (int i = 0; i < CW; i++) sm.coarse[i * BLOCK + tid] = 0;
+#pragma unroll
+            for (int i = 0; i < FW; i++) sm.fine[i * BLOCK + tid] = 0;
+            if (tid < 2) sm.mixed[tid] = 0;
+            K kmax = 0, kinv = 0;
+#pragma unroll
+            for (int j = 0; j < ITEMS; j++) {
+                key[j] = tid < n_all - j * BLOCK ? rank_key(xs[j]) : ~K(0);
+                const bool live = key[j] != ~K(0);
+                n += (uint32_t)__popcll(__ballot(live));
+                const K a = live ? key[j] : K(0), b = ~key[j];
+                kmax = a > kmax ? a : kmax;
+                kinv = b > kinv ? b : kinv; // a missing cell's is 0
+            }
+            kmax = wave_max(kmax);
+            kinv = wave_max(kinv);
+            if (lane == 0) {
+                sm.wmax[w] = kmax;
+                sm.wmin[w] = kinv;
+                sm.wn[w] = n;
+            }
+            __syncthreads();
+            // lane q < NW holds wavefront q's
+            n = lane_value(dpp_row_incl_sum(lane < NW ? sm.wn[lane] : 0u), NW - 1);
+            kmax = wave_max(lane < NW ? sm.wmax[lane] : K(0));
+            kinv = wave_max(lane < NW ? sm.wmin[lane] : K(0));
+            kmin = ~kinv;
+            if (n && kmax != kmin) {
+                const K range = kmax - kmin;
+                const int bits = sizeof(K) == 8 ? 64 - __builtin_clzll((uint64_t)range) : 32 - __builtin_clz((uint32_t)range);
+                constexpr int CB = __builtin_ctz(NC);
+                sh = bits > CB ? bits - CB : 0;
+            }
+            sh = __builtin_amdgcn_readfirstlane(sh);
+            // Missing cells go through the same instructions, adding nothing to a
+            // count of their lane's own and storing the largest pattern where the
+            // keys end with it anyway: no branch per cell.
+            // 1. coarse counts
+#pragma unroll
+            for (int j = 0; j < ITEMS; j++) {
+                const bool live = key[j] != ~K(0);
+                atomicAdd(&sm.coarse[live ? (uint32_t)((key[j] - kmin) >> sh) : (uint32_t)tid], live ? 1u : 0u);
+            }
+            __syncthreads();
+            // 2. first keys of the coarse buckets
+            {
+                uint32_t c[CW], s = 0;
+#pragma unroll
+                for (int i = 0; i < CW; i++) {
+                    c[i] = sm.coarse[tid * CW + i];
+                    s += c[i];
+                }
+                const uint32_t incl = dpp_incl_sum(s);
+                if (lane == 63) sm.wc[w] = incl;
+                __syncthreads();
+                uint32_t run = before(sm.wc, w, lane) + incl - s;
+#pragma unroll
+                for (int i = 0; i < CW; i++) {
+                    sm.coarse[tid * CW + i] = run;
+                    run += c[i];
+                }
+                if (tid == 0) sm.coarse[NC] = n;
+            }
+            __syncthreads();
+            // 3. positions, and each key's turn in its bucket
+#pragma unroll
+            for (int j = 0; j < ITEMS; j++) {
+                const K r = key[j] != ~K(0) ? key[j] - kmin : K(0);
+                const uint32_t b = (uint32_t)(r >> sh);
+                const uint32_t c0 = sm.coarse[b], c1 = sm.coarse[b + 1];
+                // the bits below the bucket's, as a 32-bit fraction of its range
+                constexpr int TOP = (int)sizeof(K) * 8 - 1;
+                const uint32_t frac = (uint32_t)(((r << 1) << (TOP - sh)) >> (TOP - 31));
+                at[j] = (2 * c0 + __umulhi(frac, 2 * (c1 - c0))) >> FSH;
+            }
+        } else {
+            // 6. What the first time left in LDS: the coarse buckets' first keys
+            // and the positions' first places. A bucket's positions, two for
+            // each of its keys, divide what was one position before. The keys
+            // are loaded again, so that the first time keeps no register for it.
+            n = lane_value(sm.n, 0);
+            sh = __builtin_amdgcn_readfirstlane(sm.sh);
+            kmin = lane_value(sm.kmin, 0);
+#pragma unroll
+            for (int j = 0; j < ITEMS; j++)
+                key[j] = tid < n_all - j * BLOCK ? rank_key(*cell_at<LIN>(src, in, rin, j * BLOCK, tid, S, blk)) : ~K(0);
+#pragma unroll
+            for (int j = 0; j < ITEMS; j++) {
+                const K r = key[j] != ~K(0) ? key[j] - kmin : K(0);
+                const uint32_t b = (uint32_t)(r >> sh);
+                const uint32_t c0 = sm.coarse[b], c1 = sm.coarse[b + 1];
+                // the bits below the bucket's, as a 32-bit fraction of its range
+                constexpr int TOP = (int)sizeof(K) * 8 - 1;
+                const uint32_t frac = (uint32_t)(((r << 1) << (TOP - sh)) >> (TOP - 31));
+                // the position, the key's fraction of it, and its bucket
+                const uint32_t full = 2 * c0 + __umulhi(frac, 2 * (c1 - c0)), p = full >> FSH;
+                uint32_t f = frac * (2 * (c1 - c0));
+                if (FSH) f = __builtin_amdgcn_alignbit(full, f, FSH);
+                const uint32_t sp = __builtin_amdgcn_alignbit(sm.fine[(p >> 1) + 1], sm.fine[p >> 1], (p & 1) * 16);
+                at[j] = (2 * (sp & 0xffffu) + __umulhi(f, 2 * ((sp >> 16) - (sp & 0xffffu)))) >> FSH;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < FW; i++) sm.fine[i * BLOCK + tid] = 0;
+            __syncthreads();
         }
 #pragma unroll
         for (int j = 0; j < ITEMS; j++) {
@@ -891,10 +935,17 @@ template <typename T, int BLOCK, int ITEMS, int FSH> struct BucketRank {
 #pragma unroll
             for (int j = 0; j < ITEMS; j++)
                 if (key[j] != ~K(0) && size(j) > DEEP) mixed = mixed || sm.key[span[j] & 0xffffu] != key[j];
-            if (__ballot(mixed) && lane == 0) sm.mixed = 1;
+            if (__ballot(mixed) && lane == 0) sm.mixed[AGAIN] = 1;
         }
         __syncthreads();
-        if (__builtin_amdgcn_readfirstlane((int)sm.mixed)) return false; // the same on every lane
+        if (__builtin_amdgcn_readfirstlane((int)sm.mixed[AGAIN])) { // the same on every lane
+            if (!AGAIN && tid == 0) {
+                sm.kmin = kmin;
+                sm.sh = sh;
+                sm.n = n;
+            }
+            return false;
+        }
         const double rn = 1.0 / (double)(int)n;
         constexpr int G = ITEMS < 16 / (int)sizeof(K) ? ITEMS : 16 / (int)sizeof(K); // keys counted side by side
 #pragma unroll
@@ -953,7 +1004,9 @@ __device__ __forceinline__ void rank_row_k(const kun_cs::View &in, const kun_cs:
         typename R::Smem r;
         __device__ Smem() {}
     } sm;
-    if (B::template row<LAY, LAY>(sm.b, in, out, S, blk, t)) return;
+    if (B::template row<LAY, LAY, false>(sm.b, in, out, S, blk, t)) return;
+    __syncthreads(); // what it left in the shared memory is there
+    if (B::template row<LAY, LAY, true>(sm.b, in, out, S, blk, t)) return;
     __syncthreads(); // the flag's readers are done with the shared memory
     if constexpr (KIND == 0) R::template row<LAY, LAY>(sm.r, in, out, S, blk, t);
     else R::row(sm.r, in, out, S, blk, t);

@@ -107,3 +107,30 @@ def test_corr_tiles(executor, S, T, n, rank_inputs):
     kr.corrWith(executor, xs, y, outs, "TS", rank_inputs=rank_inputs)
     for x, o in zip(xs, outs):
         assert_bit_exact(o, ko.corr_with(x, y, rank_inputs=rank_inputs), f"S={S} T={T} n={n}")
+
+
+def _cluster_rows(S, dt, seed):
+    """Rows that crowd few buckets: clusters beside distant values, clusters
+    within clusters (which end in the sort), with ties and missing cells."""
+    rng = np.random.default_rng(seed)
+    eps = float(np.finfo(dt).eps)
+    i = np.arange(S)
+    far = lambda x, *v: np.where(i < len(v), np.resize(v, S), x)
+    rows = [
+        far(100 * (1 + 1e-4 * rng.random(S)), 1e30),
+        far(100 * (1 + 1e-4 * rng.random(S)), -1e30, np.inf, -np.inf),
+        far(1 + eps * rng.integers(0, 3 * S, S), 1e30),                                 # neighbouring values
+        far(1 + eps * rng.integers(0, 9, S), 1e30, -1e30),                              # few of them
+        far(np.where(i % 2, 1.0, 1 + 64 * eps * rng.integers(0, S, S)), 1e30),          # half of them equal
+        far(np.where(rng.random(S) < 0.02, np.nan, -3 * (1 + 1e-5 * rng.random(S))), 1e25),
+        far(np.where(i % 2, 1 + eps * rng.integers(0, 2 * S, S), rng.random(S) * 1e4), 1e30),
+        far(1e-3 + np.where(i % 3, 0, 1e-30) * rng.random(S), 1e30, 1e-30),
+    ]
+    return np.ascontiguousarray(np.stack(rows).astype(dt))
+
+
+@pytest.mark.parametrize("module", ["cs_f32", "cs_f64"])
+@pytest.mark.parametrize("S", [67, 256, 513, 2049, 8191, 8192, 8193, 16384])
+def test_rank_clusters(executor, module, S):
+    dt = catalog.load(module)[1].dtype
+    _check(executor, module, _cluster_rows(S, dt, S), _cluster_rows(S, dt, S + 1)[::-1].copy())

@@ -1038,7 +1038,7 @@ class CompEmitter(_Lowering):
             lay = self.buf_layout(op)
             if b.kind == BUF_INPUT:
                 if lay == "1":
-                    return f"kun::row_ld(b{b.idx} + sb, start + ({row}), S32, lo)"
+                    return f"kun::row_ld(p{b.idx} + sb, {row}, S32, lo)"
                 return f"b{b.idx}[kun::at<{lay}>(A.start + ({row}), s, A.S, A.T, A.blk)]"
             if lay == "1":
                 return f"kun::row_ld(b{b.idx} + sb, {row}, S32, lo)"
@@ -1111,12 +1111,12 @@ class CompEmitter(_Lowering):
             b = self.m.buffer(op.attrs["name"])
             if self.buf_layout(op) != "1":
                 return [f"const {T} {x} = {self.src_load(op, f'i{sfx} - ({it}) + {e}')};" for e, x in enumerate(names)]
-            ptr, first = f"b{b.idx}", (f"start + i{sfx}" if b.kind == BUF_INPUT else f"i{sfx}")
+            ptr = f"p{b.idx}" if b.kind == BUF_INPUT else f"b{b.idx}"
         else:
-            ptr, first = f"m{k}", f"i{sfx}"
+            ptr = f"m{k}"
         # rows known to lie in the run: no clamp, no NaN select, the row
         # offset in a scalar register (kun::wld)
-        return [f"const unsigned ro{k} = (unsigned)({first} - ({it})) * rsz;"] + [
+        return [f"const unsigned ro{k} = (unsigned)(i{sfx} - ({it})) * rsz;"] + [
             f"const {T} {x} = kun::wld({ptr}, so, ro{k} + {e} * rsz);" for e, x in enumerate(names)]
 
     # ring reads of earlier rows hoisted to the top of the row being
@@ -1297,7 +1297,7 @@ class CompEmitter(_Lowering):
         L = []
         if self.kind == PAR:
             L.append("const int c0 = chunk_id * A.zchunk[e], nrow = (int)A.L;")
-            L.append("const int c1 = c0 + A.zchunk[e] < nrow ? c0 + A.zchunk[e] : nrow;")
+            L.append("const int c1 = A.zchunk[e] < nrow - c0 ? c0 + A.zchunk[e] : nrow;")
             L.append(f"const int rbeg = c0 - {self.halo} > 0 ? c0 - {self.halo} : 0;")
         else:
             L.append("const int c0 = 0, c1 = (int)A.L, rbeg = 0;")
@@ -1305,8 +1305,9 @@ class CompEmitter(_Lowering):
         # rows and stocks in 32-bit scalars: 64-bit compares have no scalar
         # form, and the address of a row is then two scalar products, a shift
         # and an add, the lane's part a register that never changes (a rolling
-        # sum's row: 54 -> 37 instructions)
-        L.append("const int start = (int)A.start; (void)start;")
+        # sum's row: 54 -> 37 instructions). The run's first row is part of
+        # the inputs' base addresses: only rows of the run are 32-bit, which
+        # the runtime bounds (kunrt::MAX_ROWS)
         L.append(f"const unsigned S32 = (unsigned)A.S, rsz = S32 * {self.esz}u, lo = (unsigned)lane * {self.esz}u; (void)lo; (void)rsz;")
         # window loops whose rows all lie in the run take their in-run copy
         # (kun::wld) when every byte offset of the [rows][S] buffers fits
@@ -1319,6 +1320,10 @@ class CompEmitter(_Lowering):
             L.append(f"{T} *__restrict__ stT = ({T} *)((char *)A.scratch + A.zscr[e]);")
             L.append(f"int32_t *__restrict__ istp = (int32_t *)(stT + (size_t){self.n_t - self.lds_t} * cst);")
         L.extend(self.buffer_ptrs())
+        ins = {b.idx for b in (self.m.buffer(op.attrs["name"]) for op in self.srcs if isinstance(op, Input))
+               if b.kind == BUF_INPUT and self.m.input_layout == "TS"}
+        for b in sorted(ins):
+            L.append(f"const {T} *__restrict__ p{b} = b{b} + (size_t)A.start * A.S;")
         for op in self.ext:
             k = self.idx[op]
             L.append(f"const {T} *__restrict__ m{k} = (const {T} *)A.bufs[{self.mat_buf(op)}];")

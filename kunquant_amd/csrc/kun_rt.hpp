@@ -190,6 +190,9 @@ size_t elem_size(const KunModuleDesc *m);
 size_t buffer_elems(const KunModuleDesc *m, int b, size_t S, size_t T, size_t L);
 void run_graph_host(Executor &ex, const KunModuleDesc *m, const NameMap &bufs, size_t S, size_t T,
                     size_t start, size_t L);
+// Rows of one batch run: the generated kernels count them in 32 bits, with
+// some rows to spare for what they load ahead.
+constexpr size_t MAX_ROWS = 0x7fff0000;
 // argument checks of a batch run (throws)
 void check_batch_module(const KunModuleDesc *m, size_t S, size_t T, size_t start, size_t L);
 // every node of `lay` in launch order on one stream; dev: device pointers of

@@ -731,6 +731,7 @@ void check_batch_module(const KunModuleDesc *m, size_t S, size_t T, size_t start
         throw Error("The required version in the module does not match the runtime version");
     if (m->out_layout == KUN_LAYOUT_STREAM) throw Error("Cannot run stream mode module via runGraph()");
     if (start + L > T) throw Error("Bad parameter: cur_time + length exceeds total_time");
+    if (L > MAX_ROWS) throw Error("Bad parameter: length exceeds " + std::to_string(MAX_ROWS) + " rows");
     if (m->aligned && S % (size_t)m->blocking) throw Error("num_stocks must be a multiple of blocking_len");
 }
 

@@ -2,6 +2,8 @@
 lane by lane) against the oracle: every time-series stage's outputs, from
 the oracle's values of its inputs, equal the oracle's bit for bit (NaN
 positions equal), for one chunk, one-row chunks and ragged chunks."""
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 
@@ -67,3 +69,33 @@ def test_emulated_stages_without_lds(name):
 
 def test_emulated_config2_stages_match_oracle():
     _check_module("cfg2_f32", S=20, T=200, start=0, L=200, chunks=(0, 9), seed=4)
+
+
+@pytest.mark.parametrize("name", ["simple_f32", "ops_f32", "rand40_f64"])
+def test_runs_that_start_past_32_bits_of_rows(name):
+    """The run's first row is row 2^32 + 7 of the inputs, of which only the
+    run's rows exist: every load is of one of them."""
+    ir = catalog.module_ir(name)
+    emu = EmuModule(ir)
+    dt = np.float64 if ir.dtype == "double" else np.float32
+    S, L, start = 70, 90, (1 << 32) + 7
+    d = data.ohlcv(S, L, seed=4, dtype=dt, nan_frac=0.05)
+    ins = {b.name: np.ascontiguousarray(d.get(b.name, d["close"])) for b in ir.buffers if b.kind == "INPUT"}
+    exp = OracleProgram(program_text(ir)).run(ins, S, L, 0, L, nthreads=4, temps=True)
+
+    class Far:
+        """An array as the rows from `start` on of a longer one."""
+        def __init__(self, x):
+            self.flags = x.flags
+            self.ctypes = SimpleNamespace(data=(x.ctypes.data - start * S * x.itemsize) % (1 << 64))
+
+    for st in ir.stages:
+        if st.kind != "ts":
+            continue
+        for chunk in (0, 16):
+            got = {**exp, **{k: Far(x) for k, x in ins.items()}}
+            for b in st.out_bufs:
+                got[b.name] = np.full_like(exp[b.name], 12345.0)
+            emu.run_stage(st.idx, got, S, start + L, start, L, chunk)
+            for b in st.out_bufs:
+                assert np.array_equal(got[b.name], exp[b.name], equal_nan=True), (st.idx, chunk, b.name)

@@ -105,6 +105,13 @@ def test_describe_errors():
         kr.describeGraphBatch([(mod, 64, 100, 90, 20)])
 
 
+def test_rows_past_32_bits_are_refused():
+    _, mod = catalog.load("simple_f32")
+    with pytest.raises(RuntimeError, match="length exceeds 2147418112 rows"):
+        kr.describeGraphBatch([(mod, 1, 1 << 31, 0, 1 << 31)])
+    kr.describeGraphBatch([(mod, 1, 1 << 33, 1 << 32, 260)])
+
+
 def test_module_cache_key_changes_with_each_load():
     """Caches of the runtime key by (descriptor, load serial): a library
     unloaded and loaded again (its descriptors possibly at the same

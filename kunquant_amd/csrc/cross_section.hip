@@ -1055,13 +1055,22 @@ __global__ __launch_bounds__(BLOCK, (rank_waves<T, BLOCK, ITEMS>())) void rank_s
 // The result is the sequential sum bit for bit, infinities and subnormals
 // included (a subnormal sum's unit is the smallest subnormal).
 //
-// 1024 rows of 8192 floats: 16.3 us a launch (2.1 TB/s), bound by the tiles'
+// 1024 rows of 8192 floats: 15.3 us a launch (2.2 TB/s), bound by the tiles'
 // adds and scans on the one wavefront a SIMD has; the chain on one lane per
-// row took 49.5 us. 750 rows of 5003 doubles: 15.3 us against 34.6; one row
+// row took 49.5 us. 750 rows of 5003 doubles: 13.0 us against 34.6; one row
 // per session of a pool, about 2200 stocks, summed and divided: 10.3 us
 // against 24.5.
 constexpr int CHAIN_K = 16;
 constexpr int CHAIN_TILE = 64 * CHAIN_K;
+// Lanes' cells of a row's first tile that are added one by one. The sum leaves
+// a binade with about every doubling of the cells it holds, which costs a scan
+// and a start over, some 700 clocks, where an add takes nine: short rows were
+// slower than by the chain. 1000 rows of 200 floats 9.0 us (10.7 by tiles
+// from the first cell on, 8.9 by the chain alone), of 500 9.5 (11.5, 10.6), of
+// 1000 10.8 (12.9, 13.7), of 3000 16.2 (17.9, 27.4); 20000 rows of 50 doubles
+// 31 (44, 29). 16 lanes are as good for short rows and slower for 500 to 3000
+// cells, 32 slower from 500 on.
+constexpr int CHAIN_HEAD = 8;
 
 // inclusive scan over the lanes of the runs' moves from an even (i0) and an
 // odd (i1) sum, in units
@@ -1089,13 +1098,13 @@ template <typename U> __device__ __forceinline__ U scan_units(U v) {
     return v;
 }
 
-// s plus the 64 x CHAIN_K cells of a tile, added in order (lane l holds cells
-// l * CHAIN_K .. in v); v >= +0, not NaN; s is the same on every lane
-template <typename T> __device__ __forceinline__ T add_in_order(T s, const T (&v)[CHAIN_K]) {
+// s plus the cells of a tile from lane `first` on, added in order (lane l holds
+// cells l * CHAIN_K .. in v); v >= +0, not NaN; s is the same on every lane
+template <typename T> __device__ __forceinline__ T add_in_order(T s, const T (&v)[CHAIN_K], int first) {
     using U = typename kun::Bits<T>::U;
     constexpr U LIM = U(1) << kun::Bits<T>::MANT; // units in a binade
     const int lane = threadIdx.x & 63;
-    for (int first = 0;;) {
+    for (;;) {
         const U sb = kun::to_bits(s);
         if ((sb >> kun::Bits<T>::MANT) == (U(1) << kun::Bits<T>::EXPB) - 1) return s; // infinite: stays
         const U b0 = sb & ~(LIM - 1);
@@ -1152,27 +1161,46 @@ __device__ __forceinline__ T row_sum(ChainTile<T> &tile, const kun_cs::View &in,
         }
     };
     T sum = T(0);
-    auto add = [&](const T (&x)[CHAIN_K]) {
+    auto add = [&](const T (&x)[CHAIN_K], auto head) {
 #pragma unroll
         for (int j = 0; j < CHAIN_K; j++) {
             const int e = j * 64 + lane;
             tile.cell[e / CHAIN_K * ChainTile<T>::STRIDE + e % CHAIN_K] = scale_term(x[j]);
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        int first = 0;
+        if constexpr (decltype(head)::value) {
+            const int n = (int)(S < CHAIN_HEAD * CHAIN_K ? (S + CHAIN_K - 1) / CHAIN_K : CHAIN_HEAD);
+            T g[CHAIN_K];
+#pragma unroll
+            for (int k = 0; k < CHAIN_K; k++) g[k] = tile.cell[k];
+            for (; first < n; first++) {
+                T h[CHAIN_K]; // (the last turn's is not used)
+#pragma unroll
+                for (int k = 0; k < CHAIN_K; k++) h[k] = tile.cell[(first + 1) * ChainTile<T>::STRIDE + k];
+#pragma unroll
+                for (int k = 0; k < CHAIN_K; k++) {
+                    sum = sum + g[k];
+                    g[k] = h[k];
+                }
+            }
+            if (S <= CHAIN_HEAD * CHAIN_K) return;
+        }
         T v[CHAIN_K];
 #pragma unroll
         for (int k = 0; k < CHAIN_K; k++) v[k] = tile.cell[lane * ChainTile<T>::STRIDE + k];
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        sum = add_in_order(sum, v);
+        sum = add_in_order(sum, v, first);
     };
     T x[CHAIN_K], y[CHAIN_K];
     load(x, 0);
     load(y, CHAIN_TILE);
-    for (long c0 = 0; c0 < S; c0 += 2 * CHAIN_TILE) {
-        add(x);
-        load(x, c0 + 2 * CHAIN_TILE);
-        if (c0 + CHAIN_TILE < S) add(y);
-        load(y, c0 + 3 * CHAIN_TILE);
+    add(x, std::true_type{});
+    for (long c0 = CHAIN_TILE; c0 < S; c0 += 2 * CHAIN_TILE) {
+        load(x, c0 + CHAIN_TILE);
+        add(y, std::false_type{});
+        load(y, c0 + 2 * CHAIN_TILE);
+        if (c0 + CHAIN_TILE < S) add(x, std::false_type{});
     }
     return sum;
 }

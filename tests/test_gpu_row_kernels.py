@@ -134,3 +134,11 @@ def _cluster_rows(S, dt, seed):
 def test_rank_clusters(executor, module, S):
     dt = catalog.load(module)[1].dtype
     _check(executor, module, _cluster_rows(S, dt, S), _cluster_rows(S, dt, S + 1)[::-1].copy())
+
+
+@pytest.mark.parametrize("module", ["cs_f32", "cs_f64"])
+@pytest.mark.parametrize("S", [16, 112, 113, 127, 128, 129, 144, 145, 2048, 2050, 3073, 4097])
+def test_scale_heads(executor, module, S):
+    """Rows that end in, at and after the cells added one by one."""
+    dt = catalog.load(module)[1].dtype
+    _check(executor, module, _sum_rows(S, dt, S), _sum_rows(S, dt, S + 1))

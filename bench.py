@@ -477,14 +477,15 @@ def sha256_file(path):
 
 
 def rank_kernel_name(np_dt, S):
-    """Name (as rocprofv3 prints it) of the Rank kernel for rows of S stocks."""
+    """Name (as rocprofv3 prints it) of the Rank kernel for rows of S stocks
+    from one TS buffer to another."""
     import numpy as np
     t = "float" if np_dt == np.float32 else "double"
     for lim, block, items in ((256, 256, 1), (512, 256, 2), (1024, 256, 4), (2048, 512, 4), (4096, 1024, 4),
                               (8192, 1024, 8), (16384, 1024, 16)):
         if S <= lim:
             kind = 1 if (items == 16 and t == "double") else 0  # 1: keys-only radix sort
-            return f"rank_rows<{t}, {block}, {items}, {kind}>"
+            return f"rank_rows<{t}, {block}, {items}, {kind}, 1>"
     return "rank_rows"
 
 

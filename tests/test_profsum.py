@@ -3,6 +3,9 @@ timeline arithmetic (GPU-busy fraction, kernels in flight), the VALU rate
 against the 614.4 G instr/s issue peak, and the copy-calibrated traffic."""
 import csv
 import json
+import os
+
+import numpy as np
 
 from kunquant_amd import profsum
 
@@ -77,3 +80,11 @@ def test_traffic_scaled_by_copy(tmp_path):
     assert k["kun_cs_f32_s0_k0"] == {"fetch_bytes": 1000.0 * 1024 * 2, "write_bytes": 500.0 * 1024}
     assert k["scale_sums + scale_div"] == {"fetch_bytes": 30.0 * 1024 * 2, "write_bytes": 30.0 * 1024}
     assert rec["scale_fetch"] == 2.0 and rec["scale_write"] == 1.0
+
+
+def test_bench_names_the_recorded_rank_kernel():
+    """bench.py looks the Rank kernel's counters up by name."""
+    import bench
+    for kind in ("valu", "traffic"):
+        with open(os.path.join(bench.ROOT, "profiles", f"cfg2_f32_8192x1024_{kind}.json")) as f:
+            assert bench.rank_kernel_name(np.float32, 8192) in json.load(f)["kernels"]
